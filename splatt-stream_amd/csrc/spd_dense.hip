@@ -1311,6 +1311,187 @@ k_admm_chunk(TM const * __restrict__ M, double const * __restrict__ ginv, uint32
   if(t == 0) atomicAdd(its_rows, (unsigned long long) it * (unsigned long long) (r1 - r0));
 }
 
+// ---- rows in registers, columns permuted for MFMA (R <= 64) -----------------
+//
+// The product aux = V G^{-1} of 16 rows V is run transposed, aux^T = G^{-1}
+// V^T, because the lane that then receives an entry of aux can be the one
+// that held the entry of V at the same place: lane l keeps row l % 16 and
+// the columns rl_col(s, l / 16), s < RP / 4, of every matrix. Step s of the
+// product takes V's registers s as its 4 x 16 operand as they are, and with
+// G^{-1}'s rows ordered by rl_row the result's component r of tile t is
+// register 4t + r. So an iterate never passes through LDS. Columns come in
+// neighbouring pairs: a 16-byte load of a wave covers 64 contiguous bytes of
+// each of 16 rows.
+__device__ __forceinline__ uint32_t rl_col(int s, int kk)
+{
+  return (uint32_t) (8 * (s >> 1) + 2 * kk + (s & 1));
+}
+// column of aux that row i of tile t of the transposed product computes
+__device__ __forceinline__ uint32_t rl_row(int t, int i)
+{
+  return (uint32_t) (16 * t + 8 * (i >> 3) + 2 * (i & 3) + ((i >> 2) & 1));
+}
+// pairs at any 8-byte (4-byte) boundary: rows of odd rank are not 16-byte aligned
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
+typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
+template<typename TM> struct RlPair;
+template<> struct RlPair<double> { typedef d2u type; };
+template<> struct RlPair<float> { typedef f2u type; };
+
+// the lane's columns of a row of R entries (zero past R, or when !ok)
+template<int TT, typename TM>
+__device__ __forceinline__ void
+rl_load(TM const * __restrict__ row, uint32_t R, int kk, bool ok, double (&x)[4 * TT])
+{
+  #pragma unroll
+  for(int u=0; u < 2 * TT; ++u) {
+    uint32_t const c = rl_col(2 * u, kk);
+    x[2 * u] = 0.;
+    x[2 * u + 1] = 0.;
+    if(ok && c + 1 < R) {
+      typename RlPair<TM>::type const v = *(typename RlPair<TM>::type const *) (row + c);
+      x[2 * u] = (double) v.x;
+      x[2 * u + 1] = (double) v.y;
+    } else if(ok && c < R) {
+      x[2 * u] = (double) row[c];
+    }
+  }
+}
+template<int TT>
+__device__ __forceinline__ void
+rl_store(double * __restrict__ row, uint32_t R, int kk, bool ok, double const (&x)[4 * TT])
+{
+  #pragma unroll
+  for(int u=0; u < 2 * TT; ++u) {
+    uint32_t const c = rl_col(2 * u, kk);
+    if(ok && c + 1 < R) {
+      d2u v;
+      v.x = x[2 * u];
+      v.y = x[2 * u + 1];
+      *(d2u *) (row + c) = v;
+    } else if(ok && c < R) {
+      row[c] = x[2 * u];
+    }
+  }
+}
+
+// Chunked ADMM (see k_admm_chunk) for entry-wise proximal operators, ranks up
+// to 64 and chunks of up to 64 rows: M, P and D stay in registers from the
+// first iteration to the last (one wave per 16 rows, blockDim.x / 64 waves a
+// chunk), so global memory is read and written once per solve and LDS holds
+// only G^{-1} (ranks above 32; below, its operands are registers too) and
+// the waves' sums. Bound by the FP64 MFMAs (64 cycles each per SIMD) and the
+// per-iteration reduction of the four sums. 24000 rows on average, rank 32,
+// chunks of 50: 397 to 92 us a solve (k_admm_chunk reads two LDS operands
+// per multiply-add and P, D and M from memory in every iteration).
+template<int TT, typename TM>
+__global__ void __launch_bounds__(DN_THREADS)
+k_admm_chunk_reg(TM const * __restrict__ M, double const * __restrict__ ginv,
+    double const * __restrict__ rho_p, uint64_t I, uint32_t R, uint64_t chunk,
+    double * __restrict__ P, double * __restrict__ D, int prox, double lam, uint32_t max_inner,
+    double tol, unsigned long long * __restrict__ its_rows)
+{
+  constexpr int RP = TT * 16;
+  constexpr int NS = 4 * TT;
+  constexpr bool GR = (TT <= 2);
+  __shared__ double s_g[GR ? 1 : NS * TT * 64];
+  __shared__ double s_w[2][DN_THREADS / 64][4];
+  int const lane = threadIdx.x & 63;
+  int const wave = threadIdx.x >> 6;
+  int const nw = blockDim.x >> 6;
+  int const kk = lane >> 4;
+  int const rr = lane & 15;
+  uint64_t const r0 = (uint64_t) blockIdx.x * chunk;
+  uint64_t const r1 = (r0 + chunk < I) ? r0 + chunk : I;
+  uint64_t const row = r0 + wave * 16 + rr;
+  bool const ok = row < r1;
+  double g[GR ? NS * TT : 1];
+  if constexpr (GR) {
+    #pragma unroll
+    for(int s=0; s < NS; ++s) {
+      #pragma unroll
+      for(int t=0; t < TT; ++t) g[s * TT + t] = ginv[rl_row(t, rr) * RP + rl_col(s, kk)];
+    }
+  } else {
+    for(int e=wave; e < NS * TT; e += nw) {
+      s_g[e * 64 + lane] = ginv[rl_row(e % TT, rr) * RP + rl_col(e / TT, kk)];
+    }
+    __syncthreads();
+  }
+  double m[NS], p[NS], d[NS];
+  uint64_t const off = ok ? row * R : 0;
+  rl_load<TT>(M + off, R, kk, ok, m);
+  rl_load<TT>((double const *) P + off, R, kk, ok, p);
+  rl_load<TT>((double const *) D + off, R, kk, ok, d);
+  double const rho = *rho_p;
+  double const thr = dn_prox_scalar(prox, lam, rho);
+  uint32_t valid = 0;
+  #pragma unroll
+  for(int s=0; s < NS; ++s) valid |= (ok && rl_col(s, kk) < R) ? 1u << s : 0u;
+  uint32_t it = 0;
+  while(it < max_inner) {
+    d4 acc[TT];
+    #pragma unroll
+    for(int t=0; t < TT; ++t) acc[t] = (d4) 0.;
+    #pragma unroll
+    for(int s=0; s < NS; ++s) {
+      double const v = m[s] + rho * (p[s] + d[s]);
+      #pragma unroll
+      for(int t=0; t < TT; ++t) {
+        double const a = GR ? g[GR ? s * TT + t : 0] : s_g[(s * TT + t) * 64 + lane];
+        acc[t] = mfma16(a, v, acc[t]);
+      }
+    }
+    // entries past the rank and past the chunk stay zero
+    double pn = 0., pr = 0., dr = 0., dn = 0.;
+    #pragma unroll
+    for(int s=0; s < NS; ++s) {
+      bool const in = (valid >> s) & 1u;
+      double const x = in ? acc[s / 4][s % 4] : 0.;
+      double const q = in ? dn_prox_entry(x - d[s], prox, thr) : 0.;
+      double const pd = q - x;
+      double const dd = q - p[s];
+      d[s] += pd;
+      p[s] = q;
+      pn += q * q;
+      pr += pd * pd;
+      dr += dd * dd;
+      dn += d[s] * d[s];
+    }
+    #pragma unroll
+    for(int o=32; o > 0; o >>= 1) {
+      pn += __shfl_xor(pn, o, 64);
+      pr += __shfl_xor(pr, o, 64);
+      dr += __shfl_xor(dr, o, 64);
+      dn += __shfl_xor(dn, o, 64);
+    }
+    // the sums alternate between two buffers: a wave may be one iteration
+    // ahead of another that still reads
+    double (* const w)[4] = s_w[it & 1];
+    if(lane == 0) {
+      w[wave][0] = pn;
+      w[wave][1] = pr;
+      w[wave][2] = dr;
+      w[wave][3] = dn;
+    }
+    __syncthreads();
+    double a0 = 0., a1 = 0., a2 = 0., a3 = 0.;
+    for(int k=0; k < nw; ++k) {
+      a0 += w[k][0];
+      a1 += w[k][1];
+      a2 += w[k][2];
+      a3 += w[k][3];
+    }
+    ++it;
+    if(a1 <= tol * a0 && a2 <= tol * a3) break;    // the same in every thread
+  }
+  rl_store<TT>(P + off, R, kk, ok, p);
+  rl_store<TT>(D + off, R, kk, ok, d);
+  if(threadIdx.x == 0) {
+    atomicAdd(its_rows, (unsigned long long) it * (unsigned long long) (r1 - r0));
+  }
+}
+
 // Plain product for ranks above 64: out[i,j] = sum_k In[i,k] ginv[k,j].
 template<typename TM>
 __global__ void k_apply_plain(TM const * __restrict__ In, double const * __restrict__ ginv,
@@ -2076,6 +2257,23 @@ static int admm_chunked_t(TM const * M, double const * ginv, double const * rho,
   uint64_t const nchunks = spd_cdiv(I, chunk);
   uint32_t const RP = dn_rpad(R);
   bool const sx = (prox == DN_PROX_ROWSIMP);
+  // one wave per 16 rows holds the iterates in registers: chunks of up to 64
+  // rows (the default is 50) fit a block of four waves
+  if(R <= 64 && !sx && chunk <= 64) {
+    unsigned const nt = 64u * (unsigned) spd_cdiv(chunk < I ? chunk : I, 16);
+    switch(RP / 16) {
+    case 1: hipLaunchKernelGGL((k_admm_chunk_reg<1, TM>), dim3((unsigned) nchunks), dim3(nt), 0,
+                st, M, ginv, rho, I, R, chunk, P, D, prox, lam, max_inner, tol, its_rows); break;
+    case 2: hipLaunchKernelGGL((k_admm_chunk_reg<2, TM>), dim3((unsigned) nchunks), dim3(nt), 0,
+                st, M, ginv, rho, I, R, chunk, P, D, prox, lam, max_inner, tol, its_rows); break;
+    case 3: hipLaunchKernelGGL((k_admm_chunk_reg<3, TM>), dim3((unsigned) nchunks), dim3(nt), 0,
+                st, M, ginv, rho, I, R, chunk, P, D, prox, lam, max_inner, tol, its_rows); break;
+    default: hipLaunchKernelGGL((k_admm_chunk_reg<4, TM>), dim3((unsigned) nchunks), dim3(nt), 0,
+                 st, M, ginv, rho, I, R, chunk, P, D, prox, lam, max_inner, tol, its_rows); break;
+    }
+    SPD_LAUNCH_CHECK();
+    return SPD_OK;
+  }
   if(R <= 64 && sx) {
     hipLaunchKernelGGL((k_admm_chunk<TM, true, true>), dim3((unsigned) nchunks),
         dim3(DN_THREADS), 0, st, M, ginv, RP, rho, I, R, chunk, P, D, prox, lam, max_inner, tol,

@@ -556,6 +556,48 @@ def test_admm_chunked_matches_oracle(gpu_available, prox, lam):
     assert np.allclose(D, wantD, rtol=tol, atol=tol * np.max(np.abs(wantP)))
 
 
+@pytest.mark.parametrize("I,R,chunk", [(1, 1, 50), (50, 2, 50), (51, 7, 50), (130, 16, 16),
+                                       (131, 17, 17), (200, 32, 50), (77, 33, 1),
+                                       (129, 35, 64), (260, 48, 33), (190, 64, 64),
+                                       (190, 64, 65)])
+@pytest.mark.parametrize("dtype", [0, 1])
+def test_admm_chunk_edges(gpu_available, I, R, chunk, dtype):
+    # chunks below, at and above the 16-row tiles and the 64 rows of the
+    # register kernel (65: the LDS kernel), ranks around the 16-column tiles,
+    # odd ranks (rows off 16-byte boundaries), a ragged last chunk
+    rng = np.random.default_rng(100 * R + chunk)
+    A = rng.standard_normal((3 * R, R))
+    G = A.T @ A + 0.5 * np.eye(R)
+    M = rng.standard_normal((I, R)) * 4.0
+    if dtype == 1:
+        M = M.astype(np.float32)
+    P0 = np.abs(rng.standard_normal((I, R)))
+    D0 = rng.standard_normal((I, R)) * 0.1
+    prox, lam = (3, 0.0) if R % 2 else (4, 0.3)
+    wantP, wantD, wtot = orc.admm_chunked(prox, M.astype(np.float64), P0, D0, G, chunk, 50,
+                                          1e-2, lam=lam)
+    L = ps.lib()
+    RP = _rp(R)
+    bufs = [_dev(g) for g in (G, np.ones((R, R)))]
+    arr = (C.c_void_p * 2)(*[b.ptr for b in bufs])
+    ginv, rho, info, cnt = (ps.DevBuf(n) for n in (RP * RP * 8, 8, 8, 8))
+    assert L.spd_dense_chol_inv(arr, 2, 1, R, 0.0, 1, ginv.ptr, rho.ptr, info.ptr) == 0
+    # rows past the end must stay as they are
+    guard = np.full((3, R), 7.5)
+    dM, dP, dD = _dev(M), _dev(np.vstack([P0, guard])), _dev(np.vstack([D0, guard]))
+    assert L.spd_dense_admm_chunked(dM.ptr, dtype, ginv.ptr, rho.ptr, I, R, chunk, dP.ptr,
+                                    dD.ptr, prox, C.c_double(lam), 50, C.c_double(1e-2),
+                                    cnt.ptr) == 0
+    P = dP.to_host((I + 3, R), np.float64)
+    D = dD.to_host((I + 3, R), np.float64)
+    assert int(cnt.to_host((1,), np.uint64)[0]) == wtot
+    assert np.array_equal(P[I:], guard) and np.array_equal(D[I:], guard)
+    # 50 iterations of an FP64 product of R terms: far below 1e-8 of the largest entry
+    tol = 1e-8
+    assert np.allclose(P[:I], wantP, rtol=tol, atol=tol * np.max(np.abs(wantP)))
+    assert np.allclose(D[:I], wantD, rtol=tol, atol=tol * np.max(np.abs(wantP)))
+
+
 # ---- the benchmark workloads at their own kernel instantiations -----------
 
 def test_cpd_uniform_1m_rank16_20_iterations(gpu_available):
