@@ -43,6 +43,35 @@ template<> struct VecT<float, 1> { typedef float type; };
 template<> struct VecT<double, 2> { typedef double __attribute__((ext_vector_type(2))) type; };
 template<> struct VecT<double, 1> { typedef double type; };
 
+// The same vectors in global memory: rows of a rank that is no multiple of V
+// start at any element boundary (a 16-byte load needs 4-byte alignment only).
+template<typename T, int V> struct VecU;
+template<> struct VecU<float, 4> {
+  typedef float __attribute__((ext_vector_type(4), aligned(4))) type;
+};
+template<> struct VecU<float, 1> { typedef float type; };
+template<> struct VecU<double, 2> {
+  typedef double __attribute__((ext_vector_type(2), aligned(8))) type;
+};
+template<> struct VecU<double, 1> { typedef double type; };
+
+// First column of lane c of column tile `tile` (L lanes of V columns): the
+// lane that would reach past the last column of a rank that is no multiple
+// of V takes the last V columns instead. Its first vskip() columns are then
+// also the lane's before it: both hold the same sums (stores write the same
+// bits twice), and additions to memory leave them out.
+template<int V, int L>
+__device__ __forceinline__ uint32_t vcol(uint32_t tile, uint32_t c, uint32_t R)
+{
+  uint32_t const col = (tile * L + c) * V;
+  return (V > 1 && col < R && col + V > R) ? R - V : col;
+}
+template<int V, int L>
+__device__ __forceinline__ int vskip(uint32_t tile, uint32_t c, uint32_t R)
+{
+  return (int) ((tile * L + c) * V - vcol<V, L>(tile, c, R));
+}
+
 template<typename VT> __device__ __forceinline__ VT vzero() { VT z = (VT) 0; return z; }
 
 template<typename T, int V>
@@ -51,7 +80,7 @@ vload(T const * __restrict__ base, uint32_t row, uint32_t R, uint32_t col, bool 
 {
   typedef typename VecT<T, V>::type VT;
   if(!ok) return vzero<VT>();
-  return *(VT const *) (base + (uint64_t) row * R + col);
+  return (VT) *(typename VecU<T, V>::type const *) (base + (uint64_t) row * R + col);
 }
 
 template<typename T, int V>
@@ -59,8 +88,7 @@ __device__ __forceinline__ void
 vstore(T * __restrict__ base, uint32_t row, uint32_t R, uint32_t col, bool ok,
     typename VecT<T, V>::type v)
 {
-  typedef typename VecT<T, V>::type VT;
-  if(ok) *(VT *) (base + (uint64_t) row * R + col) = v;
+  if(ok) *(typename VecU<T, V>::type *) (base + (uint64_t) row * R + col) = v;
 }
 
 __device__ __forceinline__ void vatomic(float * p, float v) { unsafeAtomicAdd(p, v); }
@@ -68,7 +96,7 @@ __device__ __forceinline__ void vatomic(double * p, double v) { unsafeAtomicAdd(
 
 template<typename T, int V>
 __device__ __forceinline__ void
-vadd_atomic(T * base, uint32_t row, uint32_t R, uint32_t col, bool ok,
+vadd_atomic(T * base, uint32_t row, uint32_t R, uint32_t col, int skip, bool ok,
     typename VecT<T, V>::type v)
 {
   if(!ok) return;
@@ -77,7 +105,9 @@ vadd_atomic(T * base, uint32_t row, uint32_t R, uint32_t col, bool ok,
     vatomic(p, v);
   } else {
     #pragma unroll
-    for(int k=0; k < V; ++k) vatomic(p + k, v[k]);
+    for(int k=0; k < V; ++k) {
+      if(k >= skip) vatomic(p + k, v[k]);
+    }
   }
 }
 
@@ -274,7 +304,8 @@ k_root_fixup(T const * __restrict__ carry, uint32_t const * __restrict__ crow,
   if(w0 >= nentries) return;                  // the whole wave leaves together
   bool const two = carry2 != nullptr;
   bool const rowst = lane == 0 && blockIdx.y == 0;
-  uint32_t const col = blockIdx.y * CW + c * V;
+  uint32_t const col = vcol<V, L>(blockIdx.y, c, R);
+  int const skip = vskip<V, L>(blockIdx.y, c, R);
   bool const cok = col < R;
   uint64_t const e0 = w0 + (uint64_t) g * EPG;
   uint32_t rw[EPG];
@@ -300,7 +331,7 @@ k_root_fixup(T const * __restrict__ carry, uint32_t const * __restrict__ crow,
           r0 = r1;
           v0 = acc;
         } else {
-          vadd_atomic<T, V>(out, r1, R, col, cok, acc);
+          vadd_atomic<T, V>(out, r1, R, col, skip, cok, acc);
         }
         first = false;
       }
@@ -335,7 +366,7 @@ k_root_fixup(T const * __restrict__ carry, uint32_t const * __restrict__ crow,
         crow2[2 * wc + 1] = ref;
       }
     } else if(g == 0) {
-      vadd_atomic<T, V>(out, ref, R, col, cok, t);
+      vadd_atomic<T, V>(out, ref, R, col, skip, cok, t);
     }
     return;
   }
@@ -367,7 +398,7 @@ k_root_fixup(T const * __restrict__ carry, uint32_t const * __restrict__ crow,
       if(rows[q] != CARRY_NONE && cok) {
         VT const sv = *(VT const *) &s_slot[wave][q][c * V];
         if(two) vstore<T, V>(carry2, (uint32_t) (2 * wc + q), R, col, cok, sv);
-        else vadd_atomic<T, V>(out, rows[q], R, col, cok, sv);
+        else vadd_atomic<T, V>(out, rows[q], R, col, skip, cok, sv);
       }
     }
     if(two && rowst) {
@@ -421,6 +452,7 @@ __global__ void __launch_bounds__(R3_WAVES * 64, sizeof(T) == 4 ? 5 : 1)
 k_root3(Root3Args<T> a)
 {
   typedef typename VecT<T, V>::type VT;
+  typedef typename VecU<T, V>::type VU;
   constexpr int G = 64 / L;
   constexpr int S = R3_WN / G;
   constexpr int CW = L * V;
@@ -453,7 +485,7 @@ k_root3(Root3Args<T> a)
   uint32_t const g = lane / L;
   uint32_t const R = a.R;
   uint32_t const rowb = R * (uint32_t) sizeof(T);
-  uint32_t const col = blockIdx.y * CW + c * V;
+  uint32_t const col = vcol<V, L>(blockIdx.y, c, R);
   bool const cok = col < R;
   // lanes past the last column read column 0 (in bounds, never stored)
   uint32_t const colb = cok ? col * (uint32_t) sizeof(T) : 0u;
@@ -639,9 +671,9 @@ k_root3(Root3Args<T> a)
         for(int j=0; j < R3_BATCH; ++j) r[j] = s_rec[wave][k + j + (k + j) / S];
         #pragma unroll
         for(int j=0; j < R3_BATCH; ++j) {
-          b[j] = *(VT const *) (Bb + (r[j].x + colb));
+          b[j] = *(VU const *) (Bb + (r[j].x + colb));
           nf[j] = !HOIST || (r[j].z & R3_FST) != 0u || (k + j == k0);
-          av[j] = nf[j] ? *(VT const *) (Ab + (r[j].y + colb)) : vzero<VT>();
+          av[j] = nf[j] ? (VT) *(VU const *) (Ab + (r[j].y + colb)) : vzero<VT>();
         }
         if constexpr (HOIST) {
           #pragma unroll
@@ -653,8 +685,8 @@ k_root3(Root3Args<T> a)
         for(uint32_t kk=k; kk < k1; ++kk) {
           uint4 const r = s_rec[wave][kk + kk / S];
           bool const nf = !HOIST || (r.z & R3_FST) != 0u || kk == k0;
-          VT const b = *(VT const *) (Bb + (r.x + colb));
-          VT const av = nf ? *(VT const *) (Ab + (r.y + colb)) : vzero<VT>();
+          VT const b = *(VU const *) (Bb + (r.x + colb));
+          VT const av = nf ? (VT) *(VU const *) (Ab + (r.y + colb)) : vzero<VT>();
           step(r, rec_val(r, kk), b, av, nf);
         }
       }
@@ -873,8 +905,7 @@ template<typename T, int V>
 __device__ __forceinline__ typename VecT<T, V>::type
 vload_c(T const * __restrict__ base, uint32_t row, uint32_t R, uint32_t colc)
 {
-  typedef typename VecT<T, V>::type VT;
-  return *(VT const *) (base + (uint64_t) row * R + colc);
+  return *(typename VecU<T, V>::type const *) (base + (uint64_t) row * R + colc);
 }
 
 // Walk positions [k0, k1) of the staged chunk: s_gid[q][k] gathered rows,
@@ -887,7 +918,7 @@ template<typename T, int NG, int KIND, int V, int L, int B>
 __device__ __forceinline__ void
 walk_range(WsArgs<T> const & a, uint32_t const (*s_gid)[WS_WN], uint32_t const * s_orow,
     int32_t const * s_osl, T const * s_val, T * hot, uint32_t nhot, uint32_t k0, uint32_t k1,
-    uint32_t c, uint32_t col, uint32_t colc, bool cok,
+    uint32_t c, uint32_t col, uint32_t colc, int skip, bool cok,
     uint32_t & r0, typename VecT<T, V>::type & v0, uint32_t & r1, typename VecT<T, V>::type & v1)
 {
   typedef typename VecT<T, V>::type VT;
@@ -922,7 +953,7 @@ walk_range(WsArgs<T> const & a, uint32_t const (*s_gid)[WS_WN], uint32_t const *
             }
           }
         } else {
-          vadd_atomic<T, V>(a.out, cur, R, col, cok, acc);
+          vadd_atomic<T, V>(a.out, cur, R, col, skip, cok, acc);
         }
       }
     };
@@ -1064,7 +1095,8 @@ k_walks(WsArgs<T> a)
   int const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   uint32_t const c = lane % L;
   uint32_t const g = lane / L;
-  uint32_t const col = blockIdx.y * CW + c * V;
+  uint32_t const col = vcol<V, L>(blockIdx.y, c, a.R);
+  int const skip = vskip<V, L>(blockIdx.y, c, a.R);
   bool const cok = col < a.R;
   uint32_t const colc = cok ? col : 0u;      // lanes past the last column read column 0
   int const d = (KIND == KIND_ROOT) ? 0 : ((KIND == KIND_LEAF) ? NL : a.depth);
@@ -1235,7 +1267,7 @@ k_walks(WsArgs<T> a)
       uint32_t r0, r1;
       VT v0 = vzero<VT>(), v1 = vzero<VT>();
       walk_range<T, NG, WALK, V, L, B>(a, s_tmp[wave], s_orow[wave], s_osl[wave], s_val[wave],
-          hot, nhot, k0, k1, c, col, colc, cok, r0, v0, r1, v1);
+          hot, nhot, k0, k1, c, col, colc, skip, cok, r0, v0, r1, v1);
       if constexpr (WALK == KIND_ROOT) {
         // The chunk's edge runs, 2 per group in position order: runs of one
         // row are summed; a run closed on both sides inside the chunk is
@@ -1310,9 +1342,10 @@ k_walks(WsArgs<T> a)
     for(uint32_t x=threadIdx.x; x < nhot * CW; x += WS_WAVES * 64) {
       uint32_t const slot = x / CW;
       uint32_t const cc = x % CW;
-      uint32_t const colx = blockIdx.y * CW + cc;
+      uint32_t const cl = cc / V;
+      uint32_t const colx = vcol<V, L>(blockIdx.y, cl, a.R) + cc % V;
       T const v = hot[x];
-      if(colx < a.R && v != (T) 0) {
+      if(colx < a.R && (int) (cc % V) >= vskip<V, L>(blockIdx.y, cl, a.R) && v != (T) 0) {
         vatomic(a.out + (uint64_t) a.hot_rows[slot] * a.R + colx, v);
       }
     }
@@ -1679,29 +1712,49 @@ static int launch_walks(WsArgs<T> a, hipStream_t st)
   return SPD_OK;
 }
 
+// Lane layout (V columns per lane, L lanes per row chunk) for a rank R:
+// 16-byte loads from V columns up, also for ranks that are no multiple of V
+// (vcol). A gather instruction costs about the same whatever its lanes
+// fetch, so 35 columns as 9 lanes of 16 move four rows an instruction where
+// one column per lane moves one (FP32, rank 35, 5M nonzeros, all three modes:
+// 623 to 365 us).
+static void lane_layout(uint32_t R, int dtype, int * V, int * L)
+{
+  if(dtype == SPD_F32 && R >= 4) {
+    uint32_t const lanes = (R + 3) / 4;
+    *V = 4;
+    *L = lanes <= 2 ? 2 : lanes <= 4 ? 4 : lanes <= 8 ? 8 : 16;
+  } else if(dtype == SPD_F64 && R >= 2) {
+    uint32_t const lanes = (R + 1) / 2;
+    *V = 2;
+    *L = lanes <= 4 ? 4 : lanes <= 8 ? 8 : lanes <= 16 ? 16 : 32;
+  } else {
+    *V = 1;
+    *L = 16;
+  }
+}
+
 template<typename T, int N, int KIND>
 static int dispatch_vl(WsArgs<T> const & a, hipStream_t st)
 {
-  uint32_t const R = a.R;
+  int V = 1, L = 16;
+  lane_layout(a.R, sizeof(T) == 4 ? SPD_F32 : SPD_F64, &V, &L);
+  if(V == 1) return launch_walks<T, N, KIND, 1, 16>(a, st);
   if constexpr (sizeof(T) == 4) {
-    if(R % 4 == 0 && R >= 8) {
-      uint32_t const lanes = R / 4;
-      if(lanes <= 2) return launch_walks<T, N, KIND, 4, 2>(a, st);
-      if(lanes <= 4) return launch_walks<T, N, KIND, 4, 4>(a, st);
-      if(lanes <= 8) return launch_walks<T, N, KIND, 4, 8>(a, st);
-      return launch_walks<T, N, KIND, 4, 16>(a, st);
+    switch(L) {
+    case 2: return launch_walks<T, N, KIND, 4, 2>(a, st);
+    case 4: return launch_walks<T, N, KIND, 4, 4>(a, st);
+    case 8: return launch_walks<T, N, KIND, 4, 8>(a, st);
+    default: return launch_walks<T, N, KIND, 4, 16>(a, st);
     }
   } else {
-    if(R % 2 == 0 && R >= 8) {
-      uint32_t const lanes = R / 2;
-      if(lanes <= 4) return launch_walks<T, N, KIND, 2, 4>(a, st);
-      if(lanes <= 8) return launch_walks<T, N, KIND, 2, 8>(a, st);
-      if(lanes <= 16) return launch_walks<T, N, KIND, 2, 16>(a, st);
-      return launch_walks<T, N, KIND, 2, 32>(a, st);
+    switch(L) {
+    case 4: return launch_walks<T, N, KIND, 2, 4>(a, st);
+    case 8: return launch_walks<T, N, KIND, 2, 8>(a, st);
+    case 16: return launch_walks<T, N, KIND, 2, 16>(a, st);
+    default: return launch_walks<T, N, KIND, 2, 32>(a, st);
     }
   }
-  if(R <= 16) return launch_walks<T, N, KIND, 1, 16>(a, st);
-  return launch_walks<T, N, KIND, 1, 64>(a, st);
 }
 
 template<typename T, int V, int L, bool HOIST>
@@ -1714,23 +1767,6 @@ static int launch_root3(Root3Args<T> const & a, uint32_t nblocks, hipStream_t st
   SPD_LAUNCH_CHECK();
   if(ev_main_end) SPD_HIP(hipEventRecord(ev_main_end, st));
   return launch_fixup<T, V, L>(a.carry, a.carry_row, 2ull * nblocks, a.out, a.R, grid.y, st);
-}
-
-// Lane layout (V columns per lane, L lanes per row chunk) for a rank R.
-static void lane_layout(uint32_t R, int dtype, int * V, int * L)
-{
-  if(dtype == SPD_F32 && R % 4 == 0 && R >= 8) {
-    uint32_t const lanes = R / 4;
-    *V = 4;
-    *L = lanes <= 2 ? 2 : lanes <= 4 ? 4 : lanes <= 8 ? 8 : 16;
-  } else if(dtype == SPD_F64 && R % 2 == 0 && R >= 8) {
-    uint32_t const lanes = R / 2;
-    *V = 2;
-    *L = lanes <= 4 ? 4 : lanes <= 8 ? 8 : lanes <= 16 ? 16 : 32;
-  } else {
-    *V = 1;
-    *L = R <= 16 ? 16 : 64;
-  }
 }
 
 template<typename T, bool HOIST>
@@ -1756,8 +1792,7 @@ static int dispatch_root3_h(Root3Args<T> const & a, uint32_t nblocks, int V, int
       }
     }
   }
-  if(L == 16) return launch_root3<T, 1, 16, HOIST>(a, nblocks, st, ev);
-  return launch_root3<T, 1, 64, HOIST>(a, nblocks, st, ev);
+  return launch_root3<T, 1, 16, HOIST>(a, nblocks, st, ev);
 }
 
 template<typename T>
@@ -2098,7 +2133,7 @@ static int run_root3(spd_csf * c, uint64_t R, void * const * mats, void * out,
   lane_layout((uint32_t) R, dtype, &V, &L);
   // the persistent kernel encodes hot rows in bit 31 of B byte offsets and
   // needs at least one chunk per wave of a full grid to pay for its LDS fill
-  if((g_root_variant == 1 || g_root_variant == 2) && root3h_layout(dtype, V, L) &&
+  if((g_root_variant == 1 || g_root_variant == 2) && root3h_layout(dtype, V, L) && R % V == 0 &&
       c->dims[c->perm[2]] * R * sizeof(T) < 0x80000000ull && c->nnz < 0xFFFFFFFFull &&
       c->nnz >= (uint64_t) R3_WN * 64) {
     return run_root3h<T>(c, R, mats, out, rows_pos, st, V, L, fx);

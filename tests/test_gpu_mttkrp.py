@@ -340,3 +340,33 @@ def test_root_kernel_variants(gpu_available, R, prec):
         finally:
             L.spd_mttkrp_set_root_variant(0)
             s.free()
+
+
+@pytest.mark.parametrize("R", [2, 4, 5, 6, 7, 9, 10, 13, 31, 33, 35, 63, 65, 67, 70])
+@pytest.mark.parametrize("prec", [ps.F64, ps.F32])
+@pytest.mark.parametrize("layout", [ps.LAYOUT_AUTO, ps.LAYOUT_CSF])
+def test_ranks_off_the_vector_width(gpu_available, R, prec, layout):
+    # ranks that are no multiple of a lane's columns: the last lane's columns
+    # overlap the lane's before it (stores and additions, one and two column
+    # tiles, root, internal and leaf outputs), and nothing is written past
+    # the last row
+    print("case odd rank", R, prec, layout, flush=True)
+    _set_layout(layout)
+    L = ps.lib()
+    dt = np.float32 if prec == ps.F32 else np.float64
+    for dims, zipf in (([90, 70, 50], [1.2, 1.1, 0.0]), ([40, 30, 20, 12], [1.2, 0.0, 1.1, 0.0])):
+        inds, vals, dims = ps.synth_coord(dims, 6000, zipf=zipf, vals="lognormal", seed=R)
+        opts = ps.Opts(csf_alloc=ps.CSF_ONEMODE)
+        s = ps.CsfSet.convert(inds, vals, opts)
+        coo = orc.Coo.from_arrays(inds, vals, dims)
+        mats = [ps.synth_matrix(d, R, 60 + m).astype(dt) for m, d in enumerate(dims)]
+        bufs = [ps.DevBuf.from_host(m) for m in mats]
+        arr = (ctypes.c_void_p * len(bufs))(*[b.ptr for b in bufs])
+        for mode, d in enumerate(dims):
+            out = ps.DevBuf.from_host(np.full((d + 2, R), 3.5, dtype=dt))
+            assert L.splatt_amd_mttkrp_dev(mode, R, s.ptr, arr, out.ptr, prec, opts.ptr,
+                                           None) == ps.SUCCESS
+            got = out.to_host((d + 2, R), dt)
+            assert np.all(got[d:] == 3.5)
+            want = orc.mttkrp_coo(coo, mats, mode, f32=(prec == ps.F32))
+            assert rel(got[:d], want) <= (TOL32 if prec == ps.F32 else TOL64)
