@@ -124,7 +124,12 @@ vadd_atomic(T * base, uint32_t row, uint32_t R, uint32_t col, int skip, bool ok,
 // id of every fiber and output row of every slice that overlaps its range.
 // Where fibers and slices start comes from two bitmaps built once per CSF
 // (one bit per nonzero: a fiber starts, a slice starts); a position's local
-// fiber and slice index is a population count over the wave's 256 bits. A group then walks its item in batches of R3_BATCH
+// fiber and slice index is a population count over the wave's 256 bits. The
+// bits at the groups' edges also tell which slices continue there, so nothing
+// is loaded after the walk, and the waves of a block keep their LDS apart
+// instead of sharing it behind a barrier (a wave holds its slot until it
+// ends: 1721 to 1497 us a step of the 50M-nonzero benchmark). A group then
+// walks its item in batches of R3_BATCH
 // nonzeros: the B row and the fiber's A row of every nonzero of a batch are
 // gathered together (2 * R3_BATCH gathers in flight), and every boundary
 // test reads LDS. k_root3h (spd_root3h.hpp) is the persistent variant that
@@ -137,7 +142,19 @@ vadd_atomic(T * base, uint32_t row, uint32_t R, uint32_t col, int skip, bool ok,
 
 #define R3_WAVES 4
 #define R3_WN 256                  // nonzeros per wave
-#define R3_BATCH 6
+// Gathers of a batch per group (each of a B and an A row), and the blocks per
+// CU that the FP32 kernels' registers are held to. A wave's time is a chain of
+// latencies (staging loads, then a gather a batch), so waves in flight count
+// more than loads a wave: 50M nonzeros, rank 32, FP32, all modes: 1497 us at
+// 6 gathers and 5 blocks, 1455 at 4 and 6 (with the long-fiber walk 1503 at 5
+// blocks, 1417 at 6).
+#define R3_BATCH 4
+#define R3_OCC 6
+// Fibers times groups in a wave's 256 nonzeros up to which it skips the A
+// gathers of steps that start no fiber in any group (at most two starts a
+// step on average): always skipping 1456 us, never 1455, this line 1417;
+// rank 35 (four groups) 360 to 335.
+#define R3_LONGF 512
 #define R3_FST 0x80000000u         // record slice field: first nonzero of a fiber
 
 // Makes v opaque to the optimiser once it is loaded. A walk that gathers A
@@ -163,8 +180,9 @@ struct Root3Args {
   T const * A;
   T const * B;
   T * out;
-  uint32_t const * plan;           // per item: slice, fiber containing its first nnz
-  uint8_t const * head;            // per item: first slice began earlier
+  uint32_t const * plan;           // slice and fiber holding the first nonzero: per wave
+                                   // (k_root3), per item (k_root3h)
+  uint8_t const * head;            // k_root3h: per item, its first slice began earlier
   uint64_t const * bits;           // per 64 nonzeros: slice-start word, fiber-start word
   T * carry;                       // 2 rows per block
   uint32_t * carry_row;
@@ -448,7 +466,7 @@ static int launch_fixup(T * carry, uint32_t * crow, uint64_t n, T * out, uint32_
 // each item) and multiplied into the slice sum at the fiber's end, as the
 // reference factors it; otherwise both rows are gathered per nonzero.
 template<typename T, int V, int L, bool HOIST>
-__global__ void __launch_bounds__(R3_WAVES * 64, sizeof(T) == 4 ? 5 : 1)
+__global__ void __launch_bounds__(R3_WAVES * 64, sizeof(T) == 4 ? R3_OCC : 1)
 k_root3(Root3Args<T> a)
 {
   typedef typename VecT<T, V>::type VT;
@@ -464,18 +482,14 @@ k_root3(Root3Args<T> a)
   // their own records fall in different LDS banks
   __shared__ uint4 s_rec[R3_WAVES][R3_WN + G];
   __shared__ T s_v64[sizeof(T) == 8 ? R3_WAVES : 1][sizeof(T) == 8 ? R3_WN + G : 1];
-  __shared__ uint32_t s_srow[R3_WAVES][R3_WN + 1];   // output row of slice S0 + k
   __shared__ uint32_t s_crow[NE];
-  // the staging-only array s_arow (A row offset of local fiber k) shares its
-  // LDS with the walk's partial rows s_cval (two per item; the block barrier
-  // between staging and walking separates the two uses). With the batch of
-  // 6 this keeps five blocks (20 waves) per CU.
-  constexpr int SZ_AROW = R3_WAVES * (R3_WN + 1) * 4;
-  constexpr int SZ_STAGE = SZ_AROW;
-  constexpr int SZ_WALK = NE * CW * (int) sizeof(T);
-  __shared__ __align__(16) unsigned char s_u[SZ_STAGE > SZ_WALK ? SZ_STAGE : SZ_WALK];
-  auto s_arow = reinterpret_cast<uint32_t (*)[R3_WN + 1]>(s_u);
-  auto s_cval = reinterpret_cast<T (*)[CW]>(s_u);
+  // output row of local slice k
+  __shared__ uint32_t s_srow[R3_WAVES][R3_WN + 1];
+  // the records' space also serves, before they are written, the A row
+  // offsets of the wave's fibers, and after the walk the items' partial rows
+  // (two per item): per wave, so that no wave waits for another
+  static_assert(2 * G * CW * sizeof(T) <= sizeof(s_rec[0]) && R3_WN * 4 <= sizeof(s_rec[0]),
+      "fiber offsets and partial rows fit in the record space");
   __shared__ uint32_t s_wrow[R3_WAVES][2];
   __shared__ __align__(16) T s_wval[R3_WAVES][2][CW];
 
@@ -490,6 +504,9 @@ k_root3(Root3Args<T> a)
   // lanes past the last column read column 0 (in bounds, never stored)
   uint32_t const colb = cok ? col * (uint32_t) sizeof(T) : 0u;
 
+  uint32_t * const s_arow = reinterpret_cast<uint32_t *>(&s_rec[wave][0]);
+  auto s_cval = reinterpret_cast<T (*)[CW]>(&s_rec[wave][0]);
+
   uint64_t const wid = (uint64_t) blockIdx.x * R3_WAVES + wave;
   uint64_t const W0 = wid * R3_WN;
   uint64_t const W1 = (W0 + R3_WN < a.nnz) ? W0 + R3_WN : a.nnz;
@@ -503,9 +520,14 @@ k_root3(Root3Args<T> a)
   // positions 1..p; local index 0 is fiber F0 (slice S0), the one holding
   // the wave's first nonzero. Each position then gets its record.
   uint32_t F0 = 0, S0 = 0;
+  // the wave's (this group's) first nonzero is not the first of its slice;
+  // the slice of its last one continues after it
+  bool whead = false, wtail = false, ghead = false, gtail = false;
+  bool longf = false;              // wave-uniform: few fibers in the wave
   if(wn > 0) {
-    S0 = a.plan[2ull * item0 + 0];
-    F0 = a.plan[2ull * item0 + 1];
+    uint2 const sf = *(uint2 const *) (a.plan + 2ull * wid);
+    S0 = sf.x;
+    F0 = sf.y;
     // this lane's PER consecutive leaf ids and values, issued first: one
     // 16-byte load each (two for FP64 values) when all PER lie in the range
     static_assert(PER == 4, "the vector staging loads assume 4 positions per lane");
@@ -543,6 +565,17 @@ k_root3(Root3Args<T> a)
     uint4 const bw = *(uint4 const *) (a.bits + 2 * (wid * 4 + (uint64_t) (lane >> 4)));
     uint64_t sw = (uint64_t) bw.x | ((uint64_t) bw.y << 32);
     uint64_t fw = (uint64_t) bw.z | ((uint64_t) bw.w << 32);
+    // a group's positions are those of its lanes: does a slice start at its
+    // first, and at the first of the next group (of the next wave)?
+    {
+      static_assert(S == PER * L, "groups stage what they walk");
+      uint64_t const nxt = (W1 < a.nnz) ? a.bits[2 * (wid * 4 + 4)] : 1ull;
+      uint32_t const first = (uint32_t) (sw >> (((uint32_t) lane & 15u) * PER)) & 1u;
+      whead = __builtin_amdgcn_readfirstlane(first) == 0u;
+      wtail = (nxt & 1ull) == 0ull;
+      ghead = __shfl((int) first, (int) (g * L), 64) == 0;
+      gtail = (g + 1 < G) ? __shfl((int) first, (int) ((g + 1) * L) & 63, 64) == 0 : wtail;
+    }
     if(lane < 16) {
       // position 0 belongs to F0 and S0 whether or not it starts them
       fw &= ~1ull;
@@ -567,11 +600,12 @@ k_root3(Root3Args<T> a)
     // fibers F0 .. F0+nfw-1 and slices S0 .. S0+nsw-1 overlap the range
     uint32_t const nfw = 1u + fc0 + fc1 + fc2 + fc3;
     uint32_t const nsw = 1u + sc0 + sc1 + sc2 + sc3;
+    longf = !HOIST && nfw * G <= R3_LONGF;
     for(uint32_t k=lane; k < nsw; k += 64) {
       s_srow[wave][k] = a.rows_are_positions ? S0 + k : a.fids0[S0 + k];
     }
     for(uint32_t k=lane; k < nfw; k += 64) {
-      s_arow[wave][k] = a.fids1[F0 + k] * rowb;
+      s_arow[k] = a.fids1[F0 + k] * rowb;
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -579,17 +613,26 @@ k_root3(Root3Args<T> a)
     uint32_t fm[PER];
     #pragma unroll
     for(int q=0; q < PER; ++q) fm[q] = (f4 >> q) & 1u;
+    // every lane has its fibers' offsets before the records overwrite them
+    uint32_t ao[PER];
     #pragma unroll
     for(int q=0; q < PER; ++q) {
       fpre += fm[q];
+      ao[q] = s_arow[fpre];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    #pragma unroll
+    for(int q=0; q < PER; ++q) {
       spre += (s4 >> q) & 1u;
       uint32_t const p = lane * PER + q;
       uint32_t const leaf = lf[q];
       T const v = lv[q];
       uint4 r;
       r.x = leaf * rowb;
-      r.y = s_arow[wave][fpre];
-      r.z = spre | ((HOIST && fm[q]) ? R3_FST : 0u);
+      r.y = ao[q];
+      r.z = spre | (fm[q] ? R3_FST : 0u);
       if constexpr (sizeof(T) == 4) {
         r.w = __float_as_uint(v);
       } else {
@@ -599,7 +642,10 @@ k_root3(Root3Args<T> a)
       s_rec[wave][p + p / S] = r;
     }
   }
-  __syncthreads();
+  // the walk reads what other lanes of the wave staged
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 
   // ---- walk this group's item ----
   // Every nonzero contributes v * B[leaf] * A[fiber row] to its slice's
@@ -614,9 +660,10 @@ k_root3(Root3Args<T> a)
   // it ends); T, the last slice when it continues past the item's end
   uint32_t hrow = CARRY_NONE, trow = CARRY_NONE;
   VT tval = vzero<VT>();
+  VT hval = vzero<VT>();
   if(n0 < a.nnz) {
     uint64_t const n1 = (n0 + S < a.nnz) ? n0 + S : a.nnz;
-    bool head_partial = a.head[item] != 0;
+    bool head_partial = ghead;
     uint32_t const k0 = (uint32_t) (n0 - W0);
     uint32_t const k1 = (uint32_t) (n1 - W0);
     uint32_t cur_s = s_rec[wave][k0 + k0 / S].z & ~R3_FST;
@@ -635,7 +682,7 @@ k_root3(Root3Args<T> a)
       uint32_t const orow = s_srow[wave][cur_s];
       if(head_partial) {
         hrow = orow;
-        if(cok) *(VT *) &s_cval[e0][c * V] = accs;
+        hval = accs;
       } else {
         vstore<T, V>(a.out, orow, R, col, cok, accs);
       }
@@ -661,7 +708,37 @@ k_root3(Root3Args<T> a)
         accs += v * (b * av);
       }
     };
-    for(uint32_t k=k0; k < k1; k += R3_BATCH) {
+    uint32_t kb = k0;
+    if(longf) {
+      // few fibers: many steps start none in any group, and the wave gathers
+      // A rows only where one does
+      for(; kb + R3_BATCH <= k1; kb += R3_BATCH) {
+        uint4 r[R3_BATCH];
+        VT b[R3_BATCH];
+        VT av[R3_BATCH];
+        #pragma unroll
+        for(int j=0; j < R3_BATCH; ++j) r[j] = s_rec[wave][kb + j + (kb + j) / S];
+        #pragma unroll
+        for(int j=0; j < R3_BATCH; ++j) b[j] = *(VU const *) (Bb + (r[j].x + colb));
+        #pragma unroll
+        for(int j=0; j < R3_BATCH; ++j) {
+          bool const nf = (r[j].z & R3_FST) != 0u || kb + j == k0;
+          av[j] = vzero<VT>();
+          if(__any(nf)) {
+            if(nf) av[j] = *(VU const *) (Ab + (r[j].y + colb));
+          }
+        }
+        #pragma unroll
+        for(int j=0; j < R3_BATCH; ++j) r3_opaque(av[j]);
+        #pragma unroll
+        for(int j=0; j < R3_BATCH; ++j) {
+          bool const nf = (r[j].z & R3_FST) != 0u || kb + j == k0;
+          if(nf) avc = av[j];
+          step(r[j], rec_val(r[j], kb + j), b[j], avc, nf);
+        }
+      }
+    }
+    for(uint32_t k=kb; k < k1; k += R3_BATCH) {
       if(k + R3_BATCH <= k1) {
         uint4 r[R3_BATCH];
         VT b[R3_BATCH];
@@ -692,22 +769,14 @@ k_root3(Root3Args<T> a)
       }
     }
     if constexpr (HOIST) accs += accf * avc;
-    // is the last slice complete at n1? It is if n1 is the start of a new
-    // slice (or the tensor's end)
-    bool complete = (n1 == a.nnz);
-    if(!complete && n1 < W1) {
-      complete = (s_rec[wave][k1 + k1 / S].z & ~R3_FST) != cur_s;
-    } else if(!complete) {
-      // the item ends at the wave's end: the slice is complete iff the
-      // next item's first slice starts there
-      complete = a.head[item + 1] == 0;
-    }
+    // the last slice is complete at n1 if a new slice (or nothing) starts there
+    bool const complete = (n1 == a.nnz) || !gtail;
     uint32_t const orow = s_srow[wave][cur_s];
     if(complete && !head_partial) {
       vstore<T, V>(a.out, orow, R, col, cok, accs);
     } else if(complete) {
       hrow = orow;
-      if(cok) *(VT *) &s_cval[e0][c * V] = accs;
+      hval = accs;
     } else {
       trow = orow;
       tval = accs;
@@ -732,12 +801,12 @@ k_root3(Root3Args<T> a)
       ref = __shfl(x, __ffsll((unsigned long long) m) - 1, 64);
       same = __all((hrow == CARRY_NONE || hrow == ref) && (trow == CARRY_NONE || trow == ref));
     }
-    bool const wopen_first = (item0 < a.nitems) && (wn > 0) && a.head[item0] != 0;
+    bool const wopen_first = whead;
     uint32_t last_item = item0 + G - 1;
     if(last_item >= a.nitems) last_item = a.nitems - 1;
     if(same) {
       VT v = vzero<VT>();
-      if(hrow != CARRY_NONE && cok) v += *(VT const *) &s_cval[e0][c * V];
+      if(hrow != CARRY_NONE) v += hval;
       if(trow != CARRY_NONE) v += tval;
       v = group_allsum<T, V, L>(v);
       // the run reaches the wave's end if the last item's T entry is in it
@@ -761,14 +830,20 @@ k_root3(Root3Args<T> a)
     } else {
       s_crow[e0] = hrow;
       s_crow[e0 + 1] = trow;
-      if(cok) *(VT *) &s_cval[e0 + 1][c * V] = tval;
+      // the records are dead once every group of the wave has walked
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      if(cok) {
+        *(VT *) &s_cval[2 * g][c * V] = hval;
+        *(VT *) &s_cval[2 * g + 1][c * V] = tval;
+      }
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
       if(g == 0) {
-        uint32_t const e_begin = wave * G * 2;
-        uint32_t const e_lastp1 = e_begin + (last_item - item0) * 2 + 1;
-        combine_runs<T, V>(s_crow, &s_cval[0][0], CW, e_begin, e_begin + 2 * G,
+        uint32_t const e_lastp1 = (last_item - item0) * 2 + 1;
+        combine_runs<T, V>(s_crow + wave * G * 2, &s_cval[0][0], CW, 0, 2 * G,
             wn > 0 ? wopen_first : false, wn > 0 ? e_lastp1 : 0xFFFFFFFFu,
             &s_wrow[wave][0], &s_wval[wave][0][0], CW, a.out, R, col, c, cok);
       }
@@ -776,8 +851,7 @@ k_root3(Root3Args<T> a)
   }
   __syncthreads();
   if(wave == 0) {
-    uint32_t const bitem0 = (uint32_t) blockIdx.x * R3_WAVES * G;
-    bool const block_head = (bitem0 < a.nitems) && a.head[bitem0] != 0;
+    bool const block_head = whead;
     // the last wave of the block with nonzeros
     uint64_t const bw0 = (uint64_t) blockIdx.x * R3_WAVES;
     uint64_t const nw_total = (a.nnz + R3_WN - 1) / R3_WN;
@@ -2138,13 +2212,11 @@ static int run_root3(spd_csf * c, uint64_t R, void * const * mats, void * out,
       c->nnz >= (uint64_t) R3_WN * 64) {
     return run_root3h<T>(c, R, mats, out, rows_pos, st, V, L, fx);
   }
-  uint32_t const G = 64 / L;
-  uint32_t const S = R3_WN / G;
   MttkrpPlan * plan = nullptr;
   if(fx == nullptr) {
-    SPD_TRY(get_plan(c, S, &plan, spd_hs(nullptr)));
+    SPD_TRY(get_plan(c, R3_WN, &plan, spd_hs(nullptr)));
     SPD_TRY(get_startbits(c, spd_hs(nullptr)));
-  } else if((plan = find_plan(c, S)) == nullptr || c->startbits == nullptr) {
+  } else if((plan = find_plan(c, R3_WN)) == nullptr || c->startbits == nullptr) {
     return not_prepared("launch plan");
   }
   if(st != spd_hs(nullptr)) {
@@ -2175,14 +2247,13 @@ static int run_root3(spd_csf * c, uint64_t R, void * const * mats, void * out,
   a.B = (T const *) mats[c->perm[2]];
   a.out = (T *) out;
   a.plan = plan->nodes;
-  a.head = plan->head;
   a.bits = c->startbits;
   a.carry = (T *) cv;
   a.carry_row = (uint32_t *) cr;
   a.nnz = c->nnz;
   a.nslices = (uint32_t) c->u.nfibs[0];
   a.nfibers = (uint32_t) c->u.nfibs[1];
-  a.nitems = plan->nitems;
+  a.nitems = (uint32_t) spd_cdiv(c->nnz, R3_WN / (64 / L));
   a.R = (uint32_t) R;
   a.rows_are_positions = rows_pos;
   SPD_TRY(spd_zero_async(out, c->dims[c->perm[0]] * R * sizeof(T), st));
