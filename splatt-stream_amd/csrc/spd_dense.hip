@@ -352,9 +352,29 @@ k_colreduce(double const * __restrict__ part, uint32_t nb, uint32_t R, uint32_t 
   b_colreduce(part, nb, R, ld, mode, lambda, out);
 }
 
+// Column norms alone (mode 0), 32 columns a block, 32 partials at a time.
+__global__ void __launch_bounds__(GR_RED_THREADS)
+k_colnorm_reduce(double const * __restrict__ part, uint32_t nb, uint32_t R, uint32_t ld,
+    double * __restrict__ out)
+{
+  __shared__ double s[GR_RED_THREADS / 32][32];
+  uint32_t const c = blockIdx.x * 32 + threadIdx.x % 32;
+  double const v = block_partsum<32, GR_RED_THREADS>(part, nb, ld, c < R, c, s);
+  if(threadIdx.x < 32 && c < R) out[c] = sqrt(v);
+}
+
 // ---- normal equations: form, Cholesky, inverse -----------------------------------
 
 struct GramSrc { double const * aTa[SPD_MAX_MODES]; };
+
+// g.aTa[m] by selection: an indexed copy of the argument would sit in memory
+__device__ __forceinline__ double const * gram_of(GramSrc const & g, int m)
+{
+  double const * p = g.aTa[0];
+  #pragma unroll
+  for(int q=1; q < SPD_MAX_MODES; ++q) p = (m == q) ? g.aTa[q] : p;
+  return p;
+}
 
 // One wave. W is 2 R^2 doubles (LDS when it fits, else global scratch).
 __global__ void __launch_bounds__(64)
@@ -439,141 +459,136 @@ k_chol_inv(GramSrc g, int nmodes, int mode, uint32_t R, uint32_t RP,
 // The same for R <= RP <= 64 by Gauss-Jordan elimination in place (no
 // pivoting: G is symmetric positive definite, and its pivots are the
 // squares of the Cholesky diagonal, so a non-positive one is reported the
-// same way). Every step updates all RP x RP entries spread over the NT
-// threads, so the work per thread is RP^3/NT independent LDS updates rather
-// than a chain of dependent ones. The result is written from its upper
-// triangle, so it is exactly symmetric.
+// same way). NT = TD^2 threads hold a W x W tile each in registers; a step
+// passes only the pivot row and column through LDS (two buffers, one barrier
+// a step; one wave up to rank 32, whose barriers are free). Bound by the
+// latency of RP dependent steps (LDS round trip, barrier, reciprocal): rank
+// 64 42.8 to 26.4 us, rank 16 6.9 to 4.5, against every entry passing through
+// LDS. The result is written from its upper triangle, so it is exactly
+// symmetric.
 template<int RP, int NT>
 __device__ __forceinline__ void
 b_gj_inv(GramSrc g, int nmodes, int mode, uint32_t R, double diag_add, int admm,
     double * __restrict__ ginv, double * __restrict__ rho_out, int * __restrict__ info)
 {
-  __shared__ double A[RP][RP + 1];
-  __shared__ double colj[RP];
-  __shared__ double s_rho;
-  constexpr int NE = RP * RP / NT;
-  static_assert(NE * NT == RP * RP && RP <= NT, "entries must split evenly");
+  constexpr int TD = (NT == 64) ? 8 : 16;
+  constexpr int W = RP / TD;
+  static_assert(TD * TD == NT && W * TD == RP, "threads tile the matrix");
+  __shared__ double s_row[2][RP];
+  __shared__ double s_col[2][RP];
   int const t = threadIdx.x;
+  int const ti = t / TD;
+  int const tj = t % TD;
   int const iR = (int) R;
-  // the Hadamard product into A, one Gram at a time in chunks of 16 entries
-  // per thread whose loads are all in flight together (the Grams were just
-  // written by other kernels and come from far away)
+  // the Hadamard product, entries past R those of the identity
+  double a[W][W];
   #pragma unroll
-  for(int q=0; q < NE; ++q) {
-    int const e = t + NT * q;
-    int const r = e / RP;
-    int const k = e - r * RP;
-    A[r][k] = (r < iR && k < iR) ? 1. : ((k == r) ? 1. : 0.);
-  }
-  constexpr int CH = (NE < 16) ? NE : 16;
-  for(int m=0; m < nmodes; ++m) {
-    if(m == mode) continue;
-    double const * const gm = g.aTa[m];
+  for(int x=0; x < W; ++x) {
     #pragma unroll
-    for(int q0=0; q0 < NE; q0 += CH) {
-      // chunks past NE (when CH does not divide NE) are skipped at compile time
-      double gv[CH];
+    for(int y=0; y < W; ++y) {
+      int const i = ti * W + x, k = tj * W + y;
+      a[x][y] = (i == k || (i < iR && k < iR)) ? 1. : 0.;
+    }
+  }
+  #pragma unroll
+  for(int m=0; m < SPD_MAX_MODES; ++m) {
+    if(m >= nmodes || m == mode) continue;     // uniform
+    double const * const gm = g.aTa[m];
+    double gv[W][W];
+    #pragma unroll
+    for(int x=0; x < W; ++x) {
       #pragma unroll
-      for(int q=0; q < CH; ++q) {
-        if(q0 + q < NE) {
-          int const e = t + NT * (q0 + q);
-          int const r = e / RP;
-          int const k = e - r * RP;
-          bool const ok = (r < iR && k < iR);
-          int const lo = r < k ? r : k;
-          int const hi = r < k ? k : r;
-          gv[q] = gm[ok ? lo * R + hi : 0];
-        }
+      for(int y=0; y < W; ++y) {
+        int const i = ti * W + x, k = tj * W + y;
+        int const lo = i < k ? i : k, hi = i < k ? k : i;
+        gv[x][y] = gm[hi < iR ? lo * R + hi : 0];
       }
+    }
+    #pragma unroll
+    for(int x=0; x < W; ++x) {
       #pragma unroll
-      for(int q=0; q < CH; ++q) {
-        if(q0 + q < NE) {
-          int const e = t + NT * (q0 + q);
-          int const r = e / RP;
-          int const k = e - r * RP;
-          A[r][k] *= (r < iR && k < iR) ? gv[q] : 1.;   // branch-free: x * 1 == x
-        }
+      for(int y=0; y < W; ++y) {
+        int const i = ti * W + x, k = tj * W + y;
+        a[x][y] *= (i < iR && k < iR) ? gv[x][y] : 1.;
       }
     }
   }
-  // the diagonal entry (t, t) belongs to another thread of the staging
-  // (in another wave when NT > 64): wait for the Hadamard product first
-  __syncthreads();
-  if(t < iR) A[t][t] += diag_add;
-  __syncthreads();
+  // the diagonal tiles' diagonal entries
+  if(ti == tj) {
+    #pragma unroll
+    for(int x=0; x < W; ++x) {
+      if(ti * W + x < iR) a[x][x] += diag_add;
+      s_row[0][ti * W + x] = a[x][x];
+    }
+  }
   if(admm) {
-    if(t == 0) {
-      double tr = 0.;
-      for(int q=0; q < iR; ++q) tr += A[q][q];
-      double const rho = tr / (double) R;
-      *rho_out = rho;
-      s_rho = rho;
+    __syncthreads();
+    double tr = 0.;
+    for(int q=0; q < iR; ++q) tr += s_row[0][q];
+    double const rho = tr / (double) R;
+    if(t == 0) *rho_out = rho;
+    if(ti == tj) {
+      #pragma unroll
+      for(int x=0; x < W; ++x) if(ti * W + x < iR) a[x][x] += rho;
     }
-    __syncthreads();
-    if(t < iR) A[t][t] += s_rho;
-    __syncthreads();
   }
+  // step 0 writes the first buffer
+  __syncthreads();
   // the first bad pivot is kept in a register and stored once at the end
   int bad = 0;
-  // Step j: colj = column j (pivot entry zeroed); row j scaled by p = 1/d
-  // with p in the pivot; column j cleared elsewhere. Then every entry takes
-  // the same update A[i][k] -= colj[i] * A[j][k]: row j passes unchanged
-  // (colj[j] = 0), column j becomes -colj[i] * p, the rest is eliminated.
-  // The update runs in chunks whose LDS reads are all issued before use.
-  constexpr int UC = (NE < 16) ? NE : 16;
-  for(int j=0; j < RP; ++j) {
-    double const d = A[j][j];
-    if(t == 0 && j < iR && !(d > 0.) && bad == 0) bad = j + 1;
-    double const p = 1. / d;
-    double cj = 0.;
-    if(t < RP) cj = A[t][j];
-    __syncthreads();
-    if(t < RP) {
-      colj[t] = (t == j) ? 0. : cj;
-      if(t == j) {
-        A[j][j] = p;
-      } else {
-        A[j][t] = A[j][t] * p;
-        A[t][j] = 0.;
-      }
-    }
-    __syncthreads();
-    // when RP divides NT a thread's entries share one column k = t % RP, so
-    // the row-j factor is read once per step (row j itself passes unchanged)
-    constexpr bool KF = (NT % RP) == 0;
-    double const ajk0 = KF ? A[j][t % RP] : 0.;
+  // Step j: with d = A[j][j], p = 1/d: row j becomes A[j][k] p, every other
+  // row loses A[i][j] times it, column j becomes -A[i][j] p, the pivot p.
+  for(int jb=0; jb < TD; ++jb) {
     #pragma unroll
-    for(int q0=0; q0 < NE; q0 += UC) {
-      double ci[UC], ajk[UC], aik[UC];
-      #pragma unroll
-      for(int q=0; q < UC; ++q) {
-        if(q0 + q < NE) {
-          int const e = t + NT * (q0 + q);
-          int const i = e / RP;
-          int const k = e - i * RP;
-          ci[q] = colj[i];
-          ajk[q] = KF ? ajk0 : A[j][k];
-          aik[q] = A[i][k];
-        }
+    for(int jj=0; jj < W; ++jj) {
+      int const j = jb * W + jj;
+      int const buf = j & 1;
+      if(ti == jb) {
+        #pragma unroll
+        for(int y=0; y < W; ++y) s_row[buf][tj * W + y] = a[jj][y];
       }
+      if(tj == jb) {
+        #pragma unroll
+        for(int x=0; x < W; ++x) s_col[buf][ti * W + x] = a[x][jj];
+      }
+      __syncthreads();
+      double const d = s_row[buf][j];
+      double r[W], c[W];
       #pragma unroll
-      for(int q=0; q < UC; ++q) {
-        if(q0 + q < NE) {
-          int const e = t + NT * (q0 + q);
-          int const i = e / RP;
-          int const k = e - i * RP;
-          A[i][k] = aik[q] - ci[q] * ajk[q];
-        }
+      for(int y=0; y < W; ++y) r[y] = s_row[buf][tj * W + y];
+      #pragma unroll
+      for(int x=0; x < W; ++x) c[x] = s_col[buf][ti * W + x];
+      if(j < iR && !(d > 0.) && bad == 0) bad = j + 1;
+      double const p = 1. / d;
+      #pragma unroll
+      for(int y=0; y < W; ++y) r[y] *= p;
+      #pragma unroll
+      for(int x=0; x < W; ++x) {
+        #pragma unroll
+        for(int y=0; y < W; ++y) a[x][y] -= c[x] * r[y];
+      }
+      if(ti == jb) {
+        #pragma unroll
+        for(int y=0; y < W; ++y) a[jj][y] = r[y];
+      }
+      if(tj == jb) {
+        #pragma unroll
+        for(int x=0; x < W; ++x) a[x][jj] = (ti == jb && x == jj) ? p : -(c[x] * p);
       }
     }
-    __syncthreads();
   }
   if(t == 0 && bad != 0 && *info == 0) *info = bad;
-  for(int e=t; e < RP * RP; e += NT) {
-    int const q = e / RP;
-    int const i = e - q * RP;
-    bool const in = (i < iR) && (q < iR);
-    ginv[e] = in ? ((q <= i) ? A[q][i] : A[i][q]) : 0.;
+  #pragma unroll
+  for(int x=0; x < W; ++x) {
+    #pragma unroll
+    for(int y=0; y < W; ++y) {
+      int const i = ti * W + x, k = tj * W + y;
+      if(i <= k) {
+        double const v = (k < iR) ? a[x][y] : 0.;
+        ginv[i * RP + k] = v;
+        ginv[k * RP + i] = v;
+      }
+    }
   }
 }
 
@@ -1375,6 +1390,89 @@ rl_store(double * __restrict__ row, uint32_t R, int kk, bool ok, double const (&
   }
 }
 
+// Product of every row with the inverse (KIND 0: X = M G^{-1}, with the
+// block's column sums of squares when colsq is given) or with a general
+// matrix (KIND 2: X += M G), ranks up to 64. A wave takes 16 rows at a time
+// in the register layout above: no row passes through LDS and no group of
+// rows waits for another. The transposed product needs G^T where G is not
+// symmetric. Rank 64, 22600 rows on average, FP32 M: 36.6 to 20.0 us; rank 16,
+// 800 rows: 8.2 to 3.6.
+template<int TT, typename TM, int KIND>
+__global__ void __launch_bounds__(DN_THREADS)
+k_apply_reg(ApplyArgs<TM> a)
+{
+  constexpr int RP = TT * 16;
+  constexpr int NS = 4 * TT;
+  constexpr bool GR = (TT <= 2);
+  __shared__ double s_g[GR ? 1 : NS * TT * 64];
+  __shared__ double s_cs[KIND == 0 ? 4 : 1][RP];
+  int const lane = threadIdx.x & 63;
+  int const wave = threadIdx.x >> 6;
+  int const kk = lane >> 4;
+  int const rr = lane & 15;
+  uint64_t const I = a.I;
+  uint32_t const R = a.R;
+  double g[GR ? NS * TT : 1];
+  // operand of step s, tile t: entry (contraction column, output column)
+  auto gent = [&](int s, int t) { return a.ginv[rl_col(s, kk) * RP + rl_row(t, rr)]; };
+  if constexpr (GR) {
+    #pragma unroll
+    for(int s=0; s < NS; ++s) {
+      #pragma unroll
+      for(int t=0; t < TT; ++t) g[s * TT + t] = gent(s, t);
+    }
+  } else {
+    for(int e=wave; e < NS * TT; e += 4) s_g[e * 64 + lane] = gent(e / TT, e % TT);
+    __syncthreads();
+  }
+  double cs[KIND == 0 ? NS : 1];
+  #pragma unroll
+  for(int s=0; s < (KIND == 0 ? NS : 1); ++s) cs[s] = 0.;
+  uint64_t const ngroups = (I + 15) / 16;
+  uint64_t const step = (uint64_t) gridDim.x * 4;
+  for(uint64_t gi = (uint64_t) blockIdx.x * 4 + wave; gi < ngroups; gi += step) {
+    uint64_t const row = gi * 16 + rr;
+    bool const ok = row < I;
+    uint64_t const off = ok ? row * R : 0;
+    double v[NS], x[NS];
+    rl_load<TT>(a.M + off, R, kk, ok, v);
+    if(KIND == 2) rl_load<TT>((double const *) a.X + off, R, kk, ok, x);
+    d4 acc[TT];
+    #pragma unroll
+    for(int t=0; t < TT; ++t) acc[t] = (d4) 0.;
+    #pragma unroll
+    for(int s=0; s < NS; ++s) {
+      #pragma unroll
+      for(int t=0; t < TT; ++t) {
+        acc[t] = mfma16(GR ? g[GR ? s * TT + t : 0] : s_g[(s * TT + t) * 64 + lane], v[s], acc[t]);
+      }
+    }
+    #pragma unroll
+    for(int s=0; s < NS; ++s) {
+      double const y = acc[s / 4][s % 4];
+      x[s] = (KIND == 2) ? x[s] + y : y;
+      // rows past the end and columns past R are zero or not stored
+      if constexpr (KIND == 0) cs[s] += ok ? y * y : 0.;
+    }
+    rl_store<TT>(a.X + off, R, kk, ok, x);
+  }
+  if constexpr (KIND == 0) {
+    if(a.colsq != nullptr) {
+      #pragma unroll
+      for(int s=0; s < NS; ++s) {
+        #pragma unroll
+        for(int o=1; o < 16; o <<= 1) cs[s] += __shfl_xor(cs[s], o, 64);
+        if(rr == 0) s_cs[wave][rl_col(s, kk)] = cs[s];
+      }
+      __syncthreads();
+      for(int e=threadIdx.x; e < RP; e += DN_THREADS) {
+        a.colsq[(uint64_t) blockIdx.x * RP + e] =
+            ((s_cs[0][e] + s_cs[1][e]) + s_cs[2][e]) + s_cs[3][e];
+      }
+    }
+  }
+}
+
 // Chunked ADMM (see k_admm_chunk) for entry-wise proximal operators, ranks up
 // to 64 and chunks of up to 64 rows: M, P and D stay in registers from the
 // first iteration to the last (one wave per 16 rows, blockDim.x / 64 waves a
@@ -1612,25 +1710,27 @@ __device__ __forceinline__ void
 b_cpd_norm(GramSrc g, int nmodes, uint32_t R,
     double const * __restrict__ lambda, double * __restrict__ out)
 {
-  __shared__ double s[64];
+  // one block of DN_THREADS: thread t sums entries t, t + DN_THREADS, ... of
+  // the upper triangle, then a fixed-order tree (one entry a thread and row
+  // took 50 us at rank 64, a row a thread)
+  __shared__ double s[DN_THREADS];
   int const t = threadIdx.x;
   double mine = 0.;
-  for(uint32_t i=t; i < R; i += 64) {
-    double row = 0.;
-    for(uint32_t j=i; j < R; ++j) {
-      double h = 1.;
-      for(int m=0; m < nmodes; ++m) h *= g.aTa[m][i * R + j];
-      row += (i == j) ? h * lambda[i] * lambda[i] : h * lambda[i] * lambda[j] * 2.;
-    }
-    mine += row;
+  for(uint32_t e=t; e < R * R; e += DN_THREADS) {
+    uint32_t const i = e / R;
+    uint32_t const j = e - i * R;
+    if(j < i) continue;
+    double h = 1.;
+    for(int m=0; m < nmodes; ++m) h *= gram_of(g, m)[e];
+    mine += (i == j) ? h * lambda[i] * lambda[i] : h * lambda[i] * lambda[j] * 2.;
   }
   s[t] = mine;
   __syncthreads();
-  if(t == 0) {
-    double tot = 0.;
-    for(int k=0; k < 64; ++k) tot += s[k];
-    out[0] = fabs(tot);
+  for(int h=DN_THREADS / 2; h > 0; h >>= 1) {
+    if(t < h) s[t] += s[t + h];
+    __syncthreads();
   }
+  if(t == 0) out[0] = fabs(s[0]);
 }
 
 __global__ void
@@ -1676,6 +1776,15 @@ int dn_div_cols(double * X, uint64_t I, uint32_t R, double const * div,
   return SPD_OK;
 }
 
+static int launch_colnorm(double const * part, uint32_t nb, uint32_t R, uint32_t ld,
+    double * out, hipStream_t st)
+{
+  hipLaunchKernelGGL(k_colnorm_reduce, dim3((unsigned) spd_cdiv(R, 32)), dim3(GR_RED_THREADS),
+      0, st, part, nb, R, ld, out);
+  SPD_LAUNCH_CHECK();
+  return SPD_OK;
+}
+
 template<typename TY, bool CLAMP>
 static int coldot(double const * X, TY const * Y, uint64_t I, uint32_t R, int mode,
     double const * lambda, double * out, hipStream_t st)
@@ -1687,6 +1796,7 @@ static int coldot(double const * X, TY const * Y, uint64_t I, uint32_t R, int mo
   hipLaunchKernelGGL((k_coldot<TY, CLAMP>), dim3(nb), dim3(DN_THREADS), 0, st,
       X, Y, I, R, rpb, (double *) part);
   SPD_LAUNCH_CHECK();
+  if(mode == 0) return launch_colnorm((double const *) part, nb, R, R, out, st);
   hipLaunchKernelGGL(k_colreduce, dim3(1), dim3(DN_THREADS), 0, st,
       (double const *) part, nb, R, R, mode, lambda, out);
   SPD_LAUNCH_CHECK();
@@ -1729,7 +1839,10 @@ static int gram_impl(double * X, double const * Y, uint64_t I, uint32_t R,
   uint32_t const TT = dn_rpad(R) / 16;
   uint32_t const RP = TT * 16;
   uint64_t const nsteps = (I + 3) / 4;
-  uint32_t const nb = dn_blocks(nsteps, 4 * GR_U * 4);
+  // two batches a wave: more, and a wave's batches (load, divide, multiply)
+  // follow each other while CUs idle (four: 26.2 us at rank 64 and 22600 rows,
+  // two: 18.0, against 6.3 and 9.1 us for summing the partials)
+  uint32_t const nb = dn_blocks(nsteps, 4 * GR_U * 2);
   void * part = nullptr;
   SPD_TRY(spd_scratch(SLOT_GRAM, (size_t) nb * RP * RP * sizeof(double), &part));
   switch(TT) {
@@ -1771,9 +1884,9 @@ int dn_chol_inv(double const * const * aTa, int nmodes, int mode, uint32_t R,
     switch(RP) {
     case 16: hipLaunchKernelGGL((k_gj_inv<16, 64>), dim3(1), dim3(64), 0, st, g, nmodes, mode,
                  R, diag_add, admm, ginv, rho, info); break;
-    case 32: hipLaunchKernelGGL((k_gj_inv<32, 128>), dim3(1), dim3(128), 0, st, g, nmodes, mode,
+    case 32: hipLaunchKernelGGL((k_gj_inv<32, 64>), dim3(1), dim3(64), 0, st, g, nmodes, mode,
                  R, diag_add, admm, ginv, rho, info); break;
-    case 48: hipLaunchKernelGGL((k_gj_inv<48, 128>), dim3(1), dim3(128), 0, st, g, nmodes, mode,
+    case 48: hipLaunchKernelGGL((k_gj_inv<48, 256>), dim3(1), dim3(256), 0, st, g, nmodes, mode,
                  R, diag_add, admm, ginv, rho, info); break;
     default: hipLaunchKernelGGL((k_gj_inv<64, 256>), dim3(1), dim3(256), 0, st, g, nmodes, mode,
                  R, diag_add, admm, ginv, rho, info); break;
@@ -1800,7 +1913,11 @@ int dn_chol_inv(double const * const * aTa, int nmodes, int mode, uint32_t R,
 template<int TT, typename TM, int KIND>
 static int launch_apply(ApplyArgs<TM> const & a, hipStream_t st, uint32_t nb)
 {
-  hipLaunchKernelGGL((k_apply_mfma<TT, TM, KIND>), dim3(nb), dim3(DN_THREADS), 0, st, a);
+  if constexpr (KIND == 1) {
+    hipLaunchKernelGGL((k_apply_mfma<TT, TM, KIND>), dim3(nb), dim3(DN_THREADS), 0, st, a);
+  } else {
+    hipLaunchKernelGGL((k_apply_reg<TT, TM, KIND>), dim3(nb), dim3(DN_THREADS), 0, st, a);
+  }
   SPD_LAUNCH_CHECK();
   return SPD_OK;
 }
@@ -1814,6 +1931,13 @@ static int dispatch_apply(ApplyArgs<TM> const & a, uint32_t TT, uint32_t nb, hip
   case 3: return launch_apply<3, TM, KIND>(a, st, nb);
   default: return launch_apply<4, TM, KIND>(a, st, nb);
   }
+}
+
+// k_apply_reg: a wave's groups of 16 rows follow each other, so as many
+// waves as there are groups, up to a resident round of blocks
+static uint32_t apply_reg_blocks(uint64_t I)
+{
+  return dn_blocks((I + 15) / 16, 4);
 }
 
 static uint32_t apply_blocks(uint64_t I)
@@ -1834,7 +1958,7 @@ static int apply_t(TM const * M, double const * ginv, uint64_t I, uint32_t R,
     if(colnorm) SPD_TRY(dn_colnorm(X, I, R, colnorm, st));
     return SPD_OK;
   }
-  uint32_t const nb = apply_blocks(I);
+  uint32_t const nb = apply_reg_blocks(I);
   void * part = nullptr;
   if(colnorm) SPD_TRY(spd_scratch(SLOT_COL, (size_t) nb * RP * sizeof(double), &part));
   ApplyArgs<TM> a = {};
@@ -1845,11 +1969,7 @@ static int apply_t(TM const * M, double const * ginv, uint64_t I, uint32_t R,
   a.X = X;
   a.colsq = (double *) part;
   SPD_TRY((dispatch_apply<TM, 0>(a, RP / 16, nb, st)));
-  if(colnorm) {
-    hipLaunchKernelGGL(k_colreduce, dim3(1), dim3(DN_THREADS), 0, st,
-        (double const *) part, nb, R, RP, 0, (double const *) nullptr, colnorm);
-    SPD_LAUNCH_CHECK();
-  }
+  if(colnorm) return launch_colnorm((double const *) part, nb, R, RP, colnorm, st);
   return SPD_OK;
 }
 
@@ -1871,7 +1991,7 @@ int dn_apply_acc(double const * In, double const * G, uint64_t I, uint32_t R,
   a.R = R;
   a.X = out;
   a.colsq = nullptr;
-  return dispatch_apply<double, 2>(a, RP / 16, apply_blocks(I), st);
+  return dispatch_apply<double, 2>(a, RP / 16, apply_reg_blocks(I), st);
 }
 
 int dn_apply(void const * M, int mdtype, double const * ginv, uint64_t I,
@@ -2061,11 +2181,7 @@ static int admm_t(TM const * M, double const * ginv, double const * rho, uint64_
     a.clamp = clamp;
     a.colsq = (double *) part;
     SPD_TRY((dispatch_apply<TM, 1>(a, RP / 16, nb, st)));
-    if(need_norms) {
-      hipLaunchKernelGGL(k_colreduce, dim3(1), dim3(DN_THREADS), 0, st,
-          (double const *) part, nb, R, RP, 0, (double const *) nullptr, norms);
-      SPD_LAUNCH_CHECK();
-    }
+    if(need_norms) SPD_TRY(launch_colnorm((double const *) part, nb, R, RP, norms, st));
   }
   if(prox == DN_PROX_SMOOTH) {
     hipLaunchKernelGGL(k_smooth_solve, dim3((unsigned) spd_cdiv(R, 64)), dim3(64), 0, st,
@@ -2321,7 +2437,7 @@ int dn_cpd_norm(double const * const * aTa, int nmodes, uint32_t R,
 {
   GramSrc g = {};
   for(int m=0; m < nmodes; ++m) g.aTa[m] = aTa[m];
-  hipLaunchKernelGGL(k_cpd_norm, dim3(1), dim3(64), 0, st, g, nmodes, R, lambda, out);
+  hipLaunchKernelGGL(k_cpd_norm, dim3(1), dim3(DN_THREADS), 0, st, g, nmodes, R, lambda, out);
   SPD_LAUNCH_CHECK();
   return SPD_OK;
 }
@@ -2789,8 +2905,8 @@ int dnb_gj_inv(uint32_t K, BSlot const * dS, BHead const * dH, uint32_t TT, int 
 {
   switch(TT) {
   case 1: hipLaunchKernelGGL((kb_gj_inv<16, 64>), dim3(K), dim3(64), 0, st, dS, dH, mode, gate); break;
-  case 2: hipLaunchKernelGGL((kb_gj_inv<32, 128>), dim3(K), dim3(128), 0, st, dS, dH, mode, gate); break;
-  case 3: hipLaunchKernelGGL((kb_gj_inv<48, 128>), dim3(K), dim3(128), 0, st, dS, dH, mode, gate); break;
+  case 2: hipLaunchKernelGGL((kb_gj_inv<32, 64>), dim3(K), dim3(64), 0, st, dS, dH, mode, gate); break;
+  case 3: hipLaunchKernelGGL((kb_gj_inv<48, 256>), dim3(K), dim3(256), 0, st, dS, dH, mode, gate); break;
   default: hipLaunchKernelGGL((kb_gj_inv<64, 256>), dim3(K), dim3(256), 0, st, dS, dH, mode, gate); break;
   }
   SPD_LAUNCH_CHECK();
@@ -2861,7 +2977,7 @@ int dnb_admm(BSlot const * hS, BSlot const * dS, BHead const * dH, uint32_t K, u
 
 int dnb_cpd_norm(uint32_t K, BSlot const * dS, BHead const * dH, hipStream_t st)
 {
-  hipLaunchKernelGGL(kb_cpd_norm, dim3(K), dim3(64), 0, st, dS, dH);
+  hipLaunchKernelGGL(kb_cpd_norm, dim3(K), dim3(DN_THREADS), 0, st, dS, dH);
   SPD_LAUNCH_CHECK();
   return SPD_OK;
 }

@@ -209,6 +209,39 @@ def test_apply(gpu_available, R, f32):
     assert np.allclose(norms, np.linalg.norm(got, axis=0), rtol=1e-12)
 
 
+@pytest.mark.parametrize("R", [1, 3, 15, 17, 32, 33, 47, 63, 64])
+@pytest.mark.parametrize("I", [1, 15, 17, 64, 257])
+@pytest.mark.parametrize("f32", [False, True])
+def test_apply_edges(gpu_available, I, R, f32):
+    # row counts around the 16-row groups and the 64 rows of a block, ranks
+    # around the 16-column tiles and off 16-byte rows; rows past the end and
+    # the inverse's padding stay out of the results
+    L = ps.lib()
+    rng = np.random.default_rng(1000 * R + I)
+    A = rng.standard_normal((3 * R, R))
+    G = A.T @ A + 0.5 * np.eye(R)
+    bufs = [_dev(G), _dev(np.ones((R, R)))]
+    arr = (C.c_void_p * 2)(*[b.ptr for b in bufs])
+    RP = _rp(R)
+    ginv, rho, info, cn = (ps.DevBuf(n) for n in (RP * RP * 8, 8, 8, R * 8))
+    assert L.spd_dense_chol_inv(arr, 2, 1, R, 0.0, 0, ginv.ptr, rho.ptr, info.ptr) == 0
+    inv = ginv.to_host((RP, RP), np.float64)
+    # G is well conditioned (a Wishart matrix plus a multiple of I)
+    assert np.allclose(inv[:R, :R] @ G, np.eye(R), atol=1e-10)
+    assert not inv[R:].any() and not inv[:, R:].any() and np.array_equal(inv, inv.T)
+    M = rng.standard_normal((I, R))
+    if f32:
+        M = M.astype(np.float32)
+    dM, X = _dev(M), _dev(np.full((I + 2, R), 4.5))
+    assert L.spd_dense_apply(dM.ptr, 1 if f32 else 0, ginv.ptr, I, R, X.ptr, cn.ptr) == 0
+    got = X.to_host((I + 2, R), np.float64)
+    assert np.all(got[I:] == 4.5)
+    # an FP64 product of R terms in another order
+    want = M.astype(np.float64) @ inv[:R, :R]
+    assert np.allclose(got[:I], want, rtol=1e-12, atol=1e-13 * np.max(np.abs(want)))
+    assert np.allclose(cn.to_host((R,), np.float64), np.linalg.norm(got[:I], axis=0), rtol=1e-12)
+
+
 @pytest.mark.parametrize("R", [8, 32, 70])
 @pytest.mark.parametrize("prox", [0, 1, 2, 3])
 def test_admm_step_matches_oracle(gpu_available, R, prox):
