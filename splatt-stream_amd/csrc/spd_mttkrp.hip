@@ -465,30 +465,34 @@ static int launch_fixup(T * carry, uint32_t * crow, uint64_t n, T * out, uint32_
 // HOIST: the fiber's A row is gathered once per fiber (and at the start of
 // each item) and multiplied into the slice sum at the fiber's end, as the
 // reference factors it; otherwise both rows are gathered per nonzero.
-template<typename T, int V, int L, bool HOIST>
+//
+// PER nonzeros a lane: a wave takes WN = 64 PER nonzeros.
+template<typename T, int V, int L, bool HOIST, int PER>
 __global__ void __launch_bounds__(R3_WAVES * 64, sizeof(T) == 4 ? R3_OCC : 1)
 k_root3(Root3Args<T> a)
 {
   typedef typename VecT<T, V>::type VT;
   typedef typename VecU<T, V>::type VU;
   constexpr int G = 64 / L;
-  constexpr int S = R3_WN / G;
+  constexpr int WN = 64 * PER;                // nonzeros per wave
+  constexpr int LPW = 64 / PER;               // lanes per bitmap word
+  constexpr int S = WN / G;
   constexpr int CW = L * V;
   constexpr int NE = R3_WAVES * G * 2;        // combine entries per block
-  constexpr int PER = R3_WN / 64;             // staged nonzeros per lane
   // per nonzero: byte offset of its B row, byte offset of its fiber's A row,
   // local slice index, and (FP32) the value's bits; FP64 values in s_v64
   // records of group g start at g * (S + 1): the groups' concurrent reads of
   // their own records fall in different LDS banks
-  __shared__ uint4 s_rec[R3_WAVES][R3_WN + G];
-  __shared__ T s_v64[sizeof(T) == 8 ? R3_WAVES : 1][sizeof(T) == 8 ? R3_WN + G : 1];
+  constexpr int NREC = (WN + G > 8 * V * (int) sizeof(T)) ? WN + G : 8 * V * (int) sizeof(T);
+  __shared__ uint4 s_rec[R3_WAVES][NREC];
+  __shared__ T s_v64[sizeof(T) == 8 ? R3_WAVES : 1][sizeof(T) == 8 ? WN + G : 1];
   __shared__ uint32_t s_crow[NE];
   // output row of local slice k
-  __shared__ uint32_t s_srow[R3_WAVES][R3_WN + 1];
+  __shared__ uint32_t s_srow[R3_WAVES][WN + 1];
   // the records' space also serves, before they are written, the A row
   // offsets of the wave's fibers, and after the walk the items' partial rows
   // (two per item): per wave, so that no wave waits for another
-  static_assert(2 * G * CW * sizeof(T) <= sizeof(s_rec[0]) && R3_WN * 4 <= sizeof(s_rec[0]),
+  static_assert(2 * G * CW * sizeof(T) <= sizeof(s_rec[0]) && WN * 4 <= sizeof(s_rec[0]),
       "fiber offsets and partial rows fit in the record space");
   __shared__ uint32_t s_wrow[R3_WAVES][2];
   __shared__ __align__(16) T s_wval[R3_WAVES][2][CW];
@@ -508,8 +512,8 @@ k_root3(Root3Args<T> a)
   auto s_cval = reinterpret_cast<T (*)[CW]>(&s_rec[wave][0]);
 
   uint64_t const wid = (uint64_t) blockIdx.x * R3_WAVES + wave;
-  uint64_t const W0 = wid * R3_WN;
-  uint64_t const W1 = (W0 + R3_WN < a.nnz) ? W0 + R3_WN : a.nnz;
+  uint64_t const W0 = wid * WN;
+  uint64_t const W1 = (W0 + WN < a.nnz) ? W0 + WN : a.nnz;
   uint32_t const item0 = (uint32_t) (wid * G);
   uint32_t const wn = (W0 < a.nnz) ? (uint32_t) (W1 - W0) : 0u;
 
@@ -530,10 +534,13 @@ k_root3(Root3Args<T> a)
     F0 = sf.y;
     // this lane's PER consecutive leaf ids and values, issued first: one
     // 16-byte load each (two for FP64 values) when all PER lie in the range
-    static_assert(PER == 4, "the vector staging loads assume 4 positions per lane");
+    static_assert(PER == 1 || PER == 4, "staging loads one or four positions per lane");
     uint32_t lf[PER];
     T lv[PER];
-    if(lane * PER + PER <= wn) {
+    if constexpr (PER == 1) {
+      lf[0] = ((uint32_t) lane < wn) ? a.leaf[W0 + lane] : 0u;
+      lv[0] = ((uint32_t) lane < wn) ? a.vals[W0 + lane] : (T) 0;
+    } else if(lane * PER + PER <= wn) {
       uint4 const l4 = *(uint4 const *) (a.leaf + W0 + lane * PER);
       lf[0] = l4.x;
       lf[1] = l4.y;
@@ -561,46 +568,53 @@ k_root3(Root3Args<T> a)
         lv[q] = (p < wn) ? a.vals[W0 + p] : (T) 0;
       }
     }
-    // this lane's slice-start and fiber-start words (16 lanes share them)
-    uint4 const bw = *(uint4 const *) (a.bits + 2 * (wid * 4 + (uint64_t) (lane >> 4)));
+    // this lane's slice-start and fiber-start words (LPW lanes share them)
+    uint4 const bw = *(uint4 const *) (a.bits + 2 * (wid * PER + (uint64_t) (lane / LPW)));
     uint64_t sw = (uint64_t) bw.x | ((uint64_t) bw.y << 32);
     uint64_t fw = (uint64_t) bw.z | ((uint64_t) bw.w << 32);
     // a group's positions are those of its lanes: does a slice start at its
     // first, and at the first of the next group (of the next wave)?
     {
       static_assert(S == PER * L, "groups stage what they walk");
-      uint64_t const nxt = (W1 < a.nnz) ? a.bits[2 * (wid * 4 + 4)] : 1ull;
-      uint32_t const first = (uint32_t) (sw >> (((uint32_t) lane & 15u) * PER)) & 1u;
+      uint64_t const nxt = (W1 < a.nnz) ? a.bits[2 * (wid + 1) * PER] : 1ull;
+      uint32_t const first = (uint32_t) (sw >> (((uint32_t) lane % LPW) * PER)) & 1u;
       whead = __builtin_amdgcn_readfirstlane(first) == 0u;
       wtail = (nxt & 1ull) == 0ull;
       ghead = __shfl((int) first, (int) (g * L), 64) == 0;
       gtail = (g + 1 < G) ? __shfl((int) first, (int) ((g + 1) * L) & 63, 64) == 0 : wtail;
     }
-    if(lane < 16) {
+    if(lane < LPW) {
       // position 0 belongs to F0 and S0 whether or not it starts them
       fw &= ~1ull;
       sw &= ~1ull;
     }
     uint32_t const fcnt = (uint32_t) __popcll(fw);
     uint32_t const scnt = (uint32_t) __popcll(sw);
-    uint32_t const fc0 = __builtin_amdgcn_readlane(fcnt, 0), fc1 = __builtin_amdgcn_readlane(fcnt, 16);
-    uint32_t const fc2 = __builtin_amdgcn_readlane(fcnt, 32), fc3 = __builtin_amdgcn_readlane(fcnt, 48);
-    uint32_t const sc0 = __builtin_amdgcn_readlane(scnt, 0), sc1 = __builtin_amdgcn_readlane(scnt, 16);
-    uint32_t const sc2 = __builtin_amdgcn_readlane(scnt, 32), sc3 = __builtin_amdgcn_readlane(scnt, 48);
-    uint32_t const wq = (uint32_t) lane >> 4;
-    uint32_t const sh = ((uint32_t) lane & 15u) * PER;
+    // counts of the wave's words (the lanes of a word agree)
+    uint32_t fc[PER], sc[PER];
+    #pragma unroll
+    for(int w=0; w < PER; ++w) {
+      fc[w] = __builtin_amdgcn_readlane(fcnt, w * LPW);
+      sc[w] = __builtin_amdgcn_readlane(scnt, w * LPW);
+    }
+    uint32_t const wq = (uint32_t) lane / LPW;
+    uint32_t const sh = ((uint32_t) lane % LPW) * PER;
     uint64_t const below = (1ull << sh) - 1ull;
-    // starts at positions before this lane's first one
-    uint32_t fpre = (wq > 0 ? fc0 : 0u) + (wq > 1 ? fc1 : 0u) + (wq > 2 ? fc2 : 0u) +
-                    (uint32_t) __popcll(fw & below);
-    uint32_t spre = (wq > 0 ? sc0 : 0u) + (wq > 1 ? sc1 : 0u) + (wq > 2 ? sc2 : 0u) +
-                    (uint32_t) __popcll(sw & below);
-    uint32_t const f4 = (uint32_t) (fw >> sh) & 15u;
-    uint32_t const s4 = (uint32_t) (sw >> sh) & 15u;
-    // fibers F0 .. F0+nfw-1 and slices S0 .. S0+nsw-1 overlap the range
-    uint32_t const nfw = 1u + fc0 + fc1 + fc2 + fc3;
-    uint32_t const nsw = 1u + sc0 + sc1 + sc2 + sc3;
-    longf = !HOIST && nfw * G <= R3_LONGF;
+    // starts at positions before this lane's first one; fibers F0 .. F0+nfw-1
+    // and slices S0 .. S0+nsw-1 overlap the range
+    uint32_t fpre = (uint32_t) __popcll(fw & below);
+    uint32_t spre = (uint32_t) __popcll(sw & below);
+    uint32_t nfw = 1u, nsw = 1u;
+    #pragma unroll
+    for(int w=0; w < PER; ++w) {
+      fpre += ((uint32_t) w < wq) ? fc[w] : 0u;
+      spre += ((uint32_t) w < wq) ? sc[w] : 0u;
+      nfw += fc[w];
+      nsw += sc[w];
+    }
+    uint32_t const f4 = (uint32_t) (fw >> sh) & ((1u << PER) - 1u);
+    uint32_t const s4 = (uint32_t) (sw >> sh) & ((1u << PER) - 1u);
+    longf = !HOIST && nfw * G * 4 <= R3_LONGF * PER;
     for(uint32_t k=lane; k < nsw; k += 64) {
       s_srow[wave][k] = a.rows_are_positions ? S0 + k : a.fids0[S0 + k];
     }
@@ -854,7 +868,7 @@ k_root3(Root3Args<T> a)
     bool const block_head = whead;
     // the last wave of the block with nonzeros
     uint64_t const bw0 = (uint64_t) blockIdx.x * R3_WAVES;
-    uint64_t const nw_total = (a.nnz + R3_WN - 1) / R3_WN;
+    uint64_t const nw_total = (a.nnz + WN - 1) / WN;
     uint32_t const lastw = (uint32_t) (((bw0 + R3_WAVES <= nw_total) ? R3_WAVES : nw_total - bw0) - 1);
     T * cv = a.carry + (uint64_t) (2 * blockIdx.x) * R;
     // the block's 2 * R3_WAVES wave slots, entry e = 2 * wave + slot; group g
@@ -1786,6 +1800,29 @@ static int launch_walks(WsArgs<T> a, hipStream_t st)
   return SPD_OK;
 }
 
+// 0: k_root3; 1: k_root3h with hot leaf rows in LDS; 2: k_root3h with
+// every row from HBM; 3: k_root3 gathering A once per fiber
+static int g_root_variant = 0;
+
+// Nonzeros a wave of k_root3 takes: 256, or 64 while 256 would leave most wave
+// slots empty and the time is one wave's chain of gathers. One mode, FP64 rank
+// 16 / FP32 rank 64, Zipf(1.1), 64 against 256: 30k nonzeros 16.1 against
+// 20.5 / 18.1 against 27.2 us, 250k 20.0 against 24.1 / 22.7 against 30.3, 500k
+// 24.8 against 25.2 / 28.3 against 31.3, 1M 32.5 against 28.9 / 36.0 against
+// 37.6 (uniform: even at 300k to 500k).
+#define R3_SMALL_NNZ 400000
+static uint64_t g_r3_small = R3_SMALL_NNZ;
+extern "C" int spd_mttkrp_set_root_small(uint64_t nnz)
+{
+  g_r3_small = nnz;
+  return SPD_OK;
+}
+
+static uint32_t root3_wn(uint64_t nnz)
+{
+  return (nnz <= g_r3_small && g_root_variant == 0) ? 64 : R3_WN;
+}
+
 // Lane layout (V columns per lane, L lanes per row chunk) for a rank R:
 // 16-byte loads from V columns up, also for ranks that are no multiple of V
 // (vcol). A gather instruction costs about the same whatever its lanes
@@ -1837,7 +1874,15 @@ static int launch_root3(Root3Args<T> const & a, uint32_t nblocks, hipStream_t st
 {
   constexpr int CW = L * V;
   dim3 grid(nblocks, (unsigned) spd_cdiv(a.R, (uint64_t) CW));
-  hipLaunchKernelGGL((k_root3<T, V, L, HOIST>), grid, dim3(R3_WAVES * 64), 0, st, a);
+  bool const small = !HOIST && root3_wn(a.nnz) == 64;
+  if constexpr (!HOIST) {
+    if(small) {
+      hipLaunchKernelGGL((k_root3<T, V, L, false, 1>), grid, dim3(R3_WAVES * 64), 0, st, a);
+    }
+  }
+  if(!small) {
+    hipLaunchKernelGGL((k_root3<T, V, L, HOIST, 4>), grid, dim3(R3_WAVES * 64), 0, st, a);
+  }
   SPD_LAUNCH_CHECK();
   if(ev_main_end) SPD_HIP(hipEventRecord(ev_main_end, st));
   return launch_fixup<T, V, L>(a.carry, a.carry_row, 2ull * nblocks, a.out, a.R, grid.y, st);
@@ -2005,10 +2050,6 @@ static int fixed_carve(MkFixed const * fx, size_t cv_bytes, size_t cr_bytes, voi
 // ---- persistent root kernel with hot leaf rows (spd_root3h.hpp) ----------
 
 #define RH_NHOT_ENC 1024           // leaf ranks encoded per CSF
-
-// 0: k_root3; 1: k_root3h with hot leaf rows in LDS; 2: k_root3h with
-// every row from HBM; 3: k_root3 gathering A once per fiber
-static int g_root_variant = 0;
 
 extern "C" int spd_mttkrp_set_root_variant(int v)
 {
@@ -2212,11 +2253,12 @@ static int run_root3(spd_csf * c, uint64_t R, void * const * mats, void * out,
       c->nnz >= (uint64_t) R3_WN * 64) {
     return run_root3h<T>(c, R, mats, out, rows_pos, st, V, L, fx);
   }
+  uint32_t const WN = root3_wn(c->nnz);
   MttkrpPlan * plan = nullptr;
   if(fx == nullptr) {
-    SPD_TRY(get_plan(c, R3_WN, &plan, spd_hs(nullptr)));
+    SPD_TRY(get_plan(c, WN, &plan, spd_hs(nullptr)));
     SPD_TRY(get_startbits(c, spd_hs(nullptr)));
-  } else if((plan = find_plan(c, R3_WN)) == nullptr || c->startbits == nullptr) {
+  } else if((plan = find_plan(c, WN)) == nullptr || c->startbits == nullptr) {
     return not_prepared("launch plan");
   }
   if(st != spd_hs(nullptr)) {
@@ -2224,7 +2266,7 @@ static int run_root3(spd_csf * c, uint64_t R, void * const * mats, void * out,
   }
   // the carry buffers belong to this call when it runs on a caller's stream
   SpdCallScratch scratch(fx ? spd_hs(nullptr) : st);
-  uint64_t const nwaves = spd_cdiv(c->nnz, R3_WN);
+  uint64_t const nwaves = spd_cdiv(c->nnz, WN);
   uint32_t const nblocks = (uint32_t) spd_cdiv(nwaves, R3_WAVES);
   // two partial rows per block, then the fix-up's second level
   uint64_t const nent = 2ull * nblocks + fix_level2_entries(2ull * nblocks);
@@ -2253,7 +2295,7 @@ static int run_root3(spd_csf * c, uint64_t R, void * const * mats, void * out,
   a.nnz = c->nnz;
   a.nslices = (uint32_t) c->u.nfibs[0];
   a.nfibers = (uint32_t) c->u.nfibs[1];
-  a.nitems = (uint32_t) spd_cdiv(c->nnz, R3_WN / (64 / L));
+  a.nitems = (uint32_t) spd_cdiv(c->nnz, WN / (64 / L));
   a.R = (uint32_t) R;
   a.rows_are_positions = rows_pos;
   SPD_TRY(spd_zero_async(out, c->dims[c->perm[0]] * R * sizeof(T), st));

@@ -370,3 +370,31 @@ def test_ranks_off_the_vector_width(gpu_available, R, prec, layout):
             assert np.all(got[d:] == 3.5)
             want = orc.mttkrp_coo(coo, mats, mode, f32=(prec == ps.F32))
             assert rel(got[:d], want) <= (TOL32 if prec == ps.F32 else TOL64)
+
+
+@pytest.mark.parametrize("small", [0, 1 << 40])
+@pytest.mark.parametrize("prec", [ps.F64, ps.F32])
+def test_slice_edges_by_wave_size(gpu_available, small, prec):
+    # both sizes of the 3-mode root kernel's waves (256 nonzeros, and the 64
+    # of small tensors) forced on the slice-edge tensor and on ranks of every
+    # lane count, with nonzeros that end inside a wave
+    L = ps.lib()
+    L.spd_mttkrp_set_root_small.argtypes = [ctypes.c_uint64]
+    assert L.spd_mttkrp_set_root_small(small) == 0
+    try:
+        test_slice_edges(gpu_available, prec, ps.LAYOUT_AUTO)
+        for R in (2, 5, 10, 16, 35, 64, 100):
+            inds, vals, dims = ps.synth_coord([70, 60, 50], 1000 + 37 * R, zipf=[1.1, 1.2, 0.0],
+                                              vals="lognormal", seed=R)
+            coo = orc.Coo.from_arrays(inds, vals, dims)
+            mats = [ps.synth_matrix(d, R, 90 + m) for m, d in enumerate(dims)]
+            m32 = [m.astype(np.float32) for m in mats]
+            s = ps.CsfSet.convert(inds, vals, ps.Opts(csf_alloc=ps.CSF_ALLMODE))
+            for mode in range(3):
+                got = s.mttkrp(mode, mats)
+                if prec == ps.F64:
+                    assert rel(got, orc.mttkrp_coo(coo, mats, mode)) <= TOL64, (R, mode)
+                else:
+                    assert rel(got, orc.mttkrp_coo(coo, m32, mode, f32=True)) <= TOL32, (R, mode)
+    finally:
+        L.spd_mttkrp_set_root_small(400000)
