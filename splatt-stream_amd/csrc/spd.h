@@ -337,6 +337,10 @@ int spd_server_close(spd_server * sv, int64_t id);
 void spd_server_stats(spd_server * sv, size_t * used, size_t * budget,
     int * admitted, int * waiting);
 void spd_server_free(spd_server * sv);
+/* n factor values from a glibc generator state, two draws each
+ * (host/base.c; used by the server's per-stream sequences). */
+struct random_data;
+void spl_fill_rand_state(struct random_data * rd, double * vals, uint64_t n);
 /* The values a server stream seeded with `seed` draws for its first n new
  * factor entries (for tests). */
 void spd_serve_rand_fill(unsigned seed, double * vals, uint64_t n);

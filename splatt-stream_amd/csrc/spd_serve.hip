@@ -101,55 +101,9 @@ struct PSlice {
   size_t off_grow[SPD_MAX_MODES] = {};
 };
 
-// n factor values from a glibc generator state (src/util.c:15-40: the
-// magnitude from one draw, the sign from the next). The draws are those of
-// random_r: for the additive feedback generator (TYPE_3, a 128-byte state)
-// the step is inlined here, with the two state pointers kept in registers
-// (random_r's own call costs several times more); other types call it.
-void fill_rand_state(struct random_data * rd, double * vals, uint64_t n)
-{
-  if(rd->rand_type != 3) {
-    for(uint64_t i=0; i < n; ++i) {
-      int32_t a = 0, b = 0;
-      random_r(rd, &a);
-      random_r(rd, &b);
-      double v = 3.0 * ((double) a / (double) RAND_MAX);
-      if(b % 2 == 0) v = -v;
-      vals[i] = v;
-    }
-    return;
-  }
-  int32_t * fptr = rd->fptr;
-  int32_t * rptr = rd->rptr;
-  int32_t * const state = rd->state;
-  int32_t * const end = rd->end_ptr;
-  auto draw = [&]() -> int32_t {
-    uint32_t const val = (uint32_t) *fptr + (uint32_t) *rptr;
-    *fptr = (int32_t) val;
-    ++fptr;
-    if(fptr >= end) {
-      fptr = state;
-      ++rptr;
-    } else {
-      ++rptr;
-      if(rptr >= end) rptr = state;
-    }
-    return (int32_t) (val >> 1);
-  };
-  for(uint64_t i=0; i < n; ++i) {
-    int32_t const a = draw();
-    int32_t const b = draw();
-    double v = 3.0 * ((double) a / (double) RAND_MAX);
-    if(b % 2 == 0) v = -v;
-    vals[i] = v;
-  }
-  rd->fptr = fptr;
-  rd->rptr = rptr;
-}
-
 void fill_stream_rand(void * ctx, double * vals, uint64_t n)
 {
-  fill_rand_state(&((Stream *) ctx)->rd, vals, n);
+  spl_fill_rand_state(&((Stream *) ctx)->rd, vals, n);
 }
 
 }  // namespace
@@ -621,7 +575,7 @@ int prepare_slice(Stream * s, Slice * sl, PSlice * ps)
   // new rows, modes in order (grow_mats)
   for(int m=0; m < N; ++m) {
     if(m == t || bd[m] <= ps->grow0[m]) continue;
-    fill_rand_state(&s->rd, (double *) (B + ps->off_grow[m]), (bd[m] - ps->grow0[m]) * R);
+    spl_fill_rand_state(&s->rd, (double *) (B + ps->off_grow[m]), (bd[m] - ps->grow0[m]) * R);
     s->prep_rows[m] = bd[m];
   }
   // the local error's mode: the smallest dim, first on ties (the streamed
@@ -1220,5 +1174,5 @@ extern "C" void spd_serve_rand_fill(unsigned seed, double * vals, uint64_t n)
   struct random_data rd = {};
   char st[128] = {};
   initstate_r(seed, st, sizeof(st), &rd);
-  fill_rand_state(&rd, vals, n);
+  spl_fill_rand_state(&rd, vals, n);
 }
