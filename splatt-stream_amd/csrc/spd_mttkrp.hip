@@ -929,8 +929,8 @@ k_root3(Root3Args<T> a)
 // CSF order keeps the nonzeros of one output-level node contiguous, so a
 // group sums a run of equal output rows in registers and flushes it once.
 //
-// A wave owns chunks of 256 consecutive nonzeros (persistent blocks stride
-// over the chunks). Per chunk it stages into LDS, with coalesced loads, the
+// A wave owns chunks of 256 consecutive nonzeros (one, or with privatised rows
+// those a persistent block strides over). Per chunk it stages into LDS, with coalesced loads, the
 // row ids and child pointers of every node of every level that overlaps the
 // chunk. Node starts are resolved bottom-up (a node starts where its first
 // child starts), marked per position and turned into local node indices with
@@ -1783,7 +1783,11 @@ static int launch_walks(WsArgs<T> a, hipStream_t st)
   constexpr int B = (N <= 4 && sizeof(T) == 8) ? 8 : 4;
   uint32_t const ny = (uint32_t) spd_cdiv(a.R, (uint64_t) CW);
   uint64_t nb = spd_cdiv(a.nchunks, WS_WAVES);
-  if(nb > WS_BLOCKS) nb = WS_BLOCKS;
+  // Blocks that privatise rows in LDS are persistent (they fill and flush
+  // them once); root and copy walks take one chunk a wave: persistent, 1024
+  // blocks were 1.3 rounds of the three a CU that FP64 registers allow
+  // (ONEMODE rank 32, 10M nonzeros, three modes: 689 to 620 us).
+  if((KIND == KIND_INTL || KIND == KIND_LEAF) && nb > WS_BLOCKS) nb = WS_BLOCKS;
   if(nb == 0) return SPD_OK;
   size_t shmem = 0;
   if constexpr (KIND == KIND_INTL || KIND == KIND_LEAF) {
