@@ -276,6 +276,88 @@ group_allsum(typename VecT<T, V>::type v)
   return v;
 }
 
+template<typename VT>
+__device__ __forceinline__ VT vshfl_up(VT v, int o)
+{
+  if constexpr (sizeof(VT) <= sizeof(double)) {
+    return __shfl_up(v, o, 64);
+  } else {
+    VT r;
+    #pragma unroll
+    for(int k=0; k < (int) (sizeof(VT) / sizeof(v[0])); ++k) r[k] = __shfl_up(v[k], o, 64);
+    return r;
+  }
+}
+
+// The edge runs of a wave's groups. Group g holds its head run (hrow, hval),
+// which ends inside the group, and its tail run (trow, tval), the group's
+// last (CARRY_NONE: none). Rows come in runs over the wave, so a tail
+// continues in the next group when that group's first run has its row; a run
+// is then the tails of some groups and a head. The tails are added along the
+// groups by a segmented scan (log2 G steps, in registers), and every run
+// finds its end in the group that holds it: it is stored, or, when it may
+// continue outside the wave, left open: the run of the last group lastg's
+// tail (slot 1), else one with the wave's first row (slot 0, open_first). The
+// group that ends an open run returns its row and sum (row0 or row1 not
+// CARRY_NONE). All of it is the groups' work side by side: a
+// serial walk over the 2G runs in LDS took longer than the nonzeros of small
+// ranks (G = 16 to 32): 8000 nonzeros at rank 10, three modes, 40.0 to 35.1 us;
+// 1.1M uniform at rank 8 114 to 88; 6.6M in four modes at rank 8 339 to 268.
+template<typename T, int V, int L>
+__device__ __forceinline__ void
+wave_runs(uint32_t hrow, typename VecT<T, V>::type hval, uint32_t trow,
+    typename VecT<T, V>::type tval, uint32_t first_row, bool open_first, uint32_t lastg,
+    T * out, uint32_t R, uint32_t col, bool cok, uint32_t & row0,
+    typename VecT<T, V>::type & val0, uint32_t & row1, typename VecT<T, V>::type & val1)
+{
+  typedef typename VecT<T, V>::type VT;
+  int const lane = threadIdx.x & 63;
+  uint32_t const g = (uint32_t) lane / L;
+  uint32_t prow = (uint32_t) __shfl_up((int) trow, L, 64);
+  if(g == 0) prow = CARRY_NONE;
+  uint32_t const own = (hrow != CARRY_NONE) ? hrow : trow;
+  uint32_t next = (uint32_t) __shfl_down((int) own, L, 64);
+  if(g == 64 / L - 1) next = CARRY_NONE;
+  // this group's tail continues the previous group's
+  bool const link = hrow == CARRY_NONE && trow != CARRY_NONE && prow == trow;
+  VT s = (trow != CARRY_NONE) ? tval : vzero<VT>();
+  int head = link ? 0 : 1;
+  #pragma unroll
+  for(int o=L; o < 64; o <<= 1) {
+    VT const up = vshfl_up(s, o);
+    int const hu = __shfl_up(head, o, 64);
+    if(lane >= o && head == 0) {
+      s += up;
+      head = hu;
+    }
+  }
+  VT const ps = vshfl_up(s, L);
+  row0 = CARRY_NONE;
+  row1 = CARRY_NONE;
+  val0 = vzero<VT>();
+  val1 = s;
+  if(hrow != CARRY_NONE) {
+    VT t = hval;
+    if(prow == hrow) t += ps;
+    if(open_first && hrow == first_row) {
+      row0 = hrow;
+      val0 = t;
+    } else {
+      vstore<T, V>(out, hrow, R, col, cok, t);
+    }
+  }
+  if(trow != CARRY_NONE && (g == lastg || next != trow)) {
+    if(g == lastg) {
+      row1 = trow;
+    } else if(open_first && trow == first_row) {
+      row0 = trow;
+      val0 = s;
+    } else {
+      vstore<T, V>(out, trow, R, col, cok, s);
+    }
+  }
+}
+
 // Root fix-up: sums the partial rows of slices that spanned several work
 // ranges (carry entries, in position order: the entries of one row are
 // consecutive). One wave owns a chunk of FIX_CHUNK entries; group g of L
@@ -291,8 +373,9 @@ group_allsum(typename VecT<T, V>::type v)
 // a heavy row then sees ~4P/FIX_CHUNK^2 atomics instead of ~2P/FIX_CHUNK,
 // which long carry buffers need (atomics on one row serialise).
 #define FIX_CHUNK 64
-// carry entries from which the fix-up takes two passes
-static uint64_t g_fix_two_level = 131072;
+// carry entries from which the fix-up takes two passes (4 modes, rank 64, 10M
+// nonzeros, 78000 entries a mode: 1080 to 1055 us a step)
+static uint64_t g_fix_two_level = 65536;
 
 extern "C" int spd_mttkrp_set_fix_two_level(uint64_t entries)
 {
@@ -479,22 +562,17 @@ k_root3(Root3Args<T> a)
   constexpr int LPW = 64 / PER;               // lanes per bitmap word
   constexpr int S = WN / G;
   constexpr int CW = L * V;
-  constexpr int NE = R3_WAVES * G * 2;        // combine entries per block
   // per nonzero: byte offset of its B row, byte offset of its fiber's A row,
   // local slice index, and (FP32) the value's bits; FP64 values in s_v64
   // records of group g start at g * (S + 1): the groups' concurrent reads of
   // their own records fall in different LDS banks
-  constexpr int NREC = (WN + G > 8 * V * (int) sizeof(T)) ? WN + G : 8 * V * (int) sizeof(T);
-  __shared__ uint4 s_rec[R3_WAVES][NREC];
+  __shared__ uint4 s_rec[R3_WAVES][WN + G];
   __shared__ T s_v64[sizeof(T) == 8 ? R3_WAVES : 1][sizeof(T) == 8 ? WN + G : 1];
-  __shared__ uint32_t s_crow[NE];
   // output row of local slice k
   __shared__ uint32_t s_srow[R3_WAVES][WN + 1];
-  // the records' space also serves, before they are written, the A row
-  // offsets of the wave's fibers, and after the walk the items' partial rows
-  // (two per item): per wave, so that no wave waits for another
-  static_assert(2 * G * CW * sizeof(T) <= sizeof(s_rec[0]) && WN * 4 <= sizeof(s_rec[0]),
-      "fiber offsets and partial rows fit in the record space");
+  // before they are written, the records' space holds the A row offsets of
+  // the wave's fibers; every wave keeps to its own, so none waits for another
+  static_assert(WN * 4 <= (int) sizeof(s_rec[0]), "fiber offsets fit in the record space");
   __shared__ uint32_t s_wrow[R3_WAVES][2];
   __shared__ __align__(16) T s_wval[R3_WAVES][2][CW];
 
@@ -510,7 +588,6 @@ k_root3(Root3Args<T> a)
   uint32_t const colb = cok ? col * (uint32_t) sizeof(T) : 0u;
 
   uint32_t * const s_arow = reinterpret_cast<uint32_t *>(&s_rec[wave][0]);
-  auto s_cval = reinterpret_cast<T (*)[CW]>(&s_rec[wave][0]);
 
   uint64_t const wid = (uint64_t) blockIdx.x * R3_WAVES + wave;
   uint64_t const W0 = wid * WN;
@@ -667,7 +744,6 @@ k_root3(Root3Args<T> a)
   // accumulator; a change of local slice flushes the finished slice.
   uint32_t const item = item0 + g;
   uint64_t const n0 = (uint64_t) item * S;
-  uint32_t const e0 = (wave * G + g) * 2;
   char const * const Bb = (char const *) a.B;
   char const * const Ab = (char const *) a.A;
   // the item's partial slices: H, the first slice when it began before the
@@ -798,70 +874,29 @@ k_root3(Root3Args<T> a)
     }
   }
   // ---- combine partial slices: per wave, then per block ----
-  // Entries (H and T of every item) are in nonzero order, so one slice's
-  // entries are adjacent. A run (entries of one row) that may continue past
-  // an edge is kept open; a run closed on both sides is complete and stored.
-  // Open runs of a wave go to its two wave slots (slot 1 if the run reaches
-  // the wave's end, slot 0 if it began before the wave), and the block
-  // combines the wave slots the same way into its two carry rows. When all
-  // of a level's entries belong to one row (a wave inside one long slice, the
-  // common case) they form a single run, summed across groups in registers;
-  // otherwise the entries go through LDS to a serial walk over the runs.
+  // A run (the partial sums of one slice) that may continue past an edge is
+  // kept open; a run closed on both sides is complete and stored. A wave's
+  // open runs go to its two slots (slot 1 if the run reaches the wave's end,
+  // slot 0 if it began before the wave), and the block combines the wave
+  // slots the same way into its two carry rows.
   {
-    uint32_t const x = (hrow != CARRY_NONE) ? hrow : trow;
-    uint64_t const m = __ballot(x != CARRY_NONE);
-    uint32_t ref = CARRY_NONE;
-    bool same = true;
-    if(m != 0) {
-      ref = __shfl(x, __ffsll((unsigned long long) m) - 1, 64);
-      same = __all((hrow == CARRY_NONE || hrow == ref) && (trow == CARRY_NONE || trow == ref));
-    }
-    bool const wopen_first = whead;
     uint32_t last_item = item0 + G - 1;
     if(last_item >= a.nitems) last_item = a.nitems - 1;
-    if(same) {
-      VT v = vzero<VT>();
-      if(hrow != CARRY_NONE) v += hval;
-      if(trow != CARRY_NONE) v += tval;
-      v = group_allsum<T, V, L>(v);
-      // the run reaches the wave's end if the last item's T entry is in it
-      uint32_t const tlast = (wn > 0) ? __shfl(trow, (int) ((last_item - item0) * L), 64) : CARRY_NONE;
-      uint32_t r0 = CARRY_NONE, r1 = CARRY_NONE;
-      if(m != 0) {
-        if(tlast != CARRY_NONE) r1 = ref;
-        else if(wopen_first) r0 = ref;
-      }
-      if(g == 0) {
-        if(r1 != CARRY_NONE) {
-          if(cok) *(VT *) &s_wval[wave][1][c * V] = v;
-        } else if(r0 != CARRY_NONE) {
-          if(cok) *(VT *) &s_wval[wave][0][c * V] = v;
-        } else if(m != 0) {
-          vstore<T, V>(a.out, ref, R, col, cok, v);
-        }
-        s_wrow[wave][0] = r0;
-        s_wrow[wave][1] = r1;
-      }
-    } else {
-      s_crow[e0] = hrow;
-      s_crow[e0 + 1] = trow;
-      // the records are dead once every group of the wave has walked
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      if(cok) {
-        *(VT *) &s_cval[2 * g][c * V] = hval;
-        *(VT *) &s_cval[2 * g + 1][c * V] = tval;
-      }
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      if(g == 0) {
-        uint32_t const e_lastp1 = (last_item - item0) * 2 + 1;
-        combine_runs<T, V>(s_crow + wave * G * 2, &s_cval[0][0], CW, 0, 2 * G,
-            wn > 0 ? wopen_first : false, wn > 0 ? e_lastp1 : 0xFFFFFFFFu,
-            &s_wrow[wave][0], &s_wval[wave][0][0], CW, a.out, R, col, c, cok);
-      }
+    uint32_t const first_row = (wn > 0) ? s_srow[wave][0] : CARRY_NONE;
+    uint32_t r0, r1;
+    VT v0, v1;
+    wave_runs<T, V, L>(hrow, hval, trow, tval, first_row, whead, last_item - item0, a.out, R, col,
+        cok, r0, v0, r1, v1);
+    bool const none0 = __ballot(r0 != CARRY_NONE) == 0, none1 = __ballot(r1 != CARRY_NONE) == 0;
+    if(lane == 0 && none0) s_wrow[wave][0] = CARRY_NONE;
+    if(lane == 0 && none1) s_wrow[wave][1] = CARRY_NONE;
+    if(r0 != CARRY_NONE) {
+      s_wrow[wave][0] = r0;
+      if(cok) *(VT *) &s_wval[wave][0][c * V] = v0;
+    }
+    if(r1 != CARRY_NONE) {
+      s_wrow[wave][1] = r1;
+      if(cok) *(VT *) &s_wval[wave][1][c * V] = v1;
     }
   }
   __syncthreads();
@@ -1369,73 +1404,35 @@ k_walks(WsArgs<T> a)
       walk_range<T, NG, WALK, V, L, B>(a, s_tmp[wave], s_orow[wave], s_osl[wave], s_val[wave],
           hot, nhot, k0, k1, c, col, colc, skip, cok, r0, v0, r1, v1);
       if constexpr (WALK == KIND_ROOT) {
-        // The chunk's edge runs, 2 per group in position order: runs of one
-        // row are summed; a run closed on both sides inside the chunk is
-        // complete and stored; the chunk's first run (it may have begun in
-        // the previous chunk) and its last run (it may continue) go to the
-        // chunk's two carry rows for k_root_fixup. Every group with
+        // The chunk's edge runs: a run closed on both sides inside the chunk
+        // is complete and stored; the chunk's first run (it may have begun
+        // in the previous chunk) and its last run (it may continue) go to
+        // the chunk's two carry rows for k_root_fixup. Every group with
         // positions ends with a last run, so the chunk's last run is always
         // carried.
-        uint32_t const x = (r0 != CARRY_NONE) ? r0 : r1;
-        uint64_t const m = __ballot(x != CARRY_NONE);
-        uint32_t ref = CARRY_NONE;
-        bool same = true;
-        if(m != 0) {
-          ref = __shfl(x, __ffsll((unsigned long long) m) - 1, 64);
-          same = __all((r0 == CARRY_NONE || r0 == ref) && (r1 == CARRY_NONE || r1 == ref));
+        T * const cv = a.carry + (uint64_t) (2 * ch) * a.R;
+        uint32_t w0, w1;
+        VT x0, x1;
+        wave_runs<T, V, L>(r0, v0, r1, v1, first_row, true, (wn + S - 1) / S - 1, a.out, a.R, col,
+            cok, w0, x0, w1, x1);
+        bool const none0 = __ballot(w0 != CARRY_NONE) == 0;
+        bool const rowst = blockIdx.y == 0;
+        if(lane == 0 && rowst && none0) a.carry_row[2 * ch] = CARRY_NONE;
+        if(w0 != CARRY_NONE) {
+          vstore<T, V>(cv, 0u, a.R, col, cok, x0);
+          if(c == 0 && rowst) a.carry_row[2 * ch] = w0;
         }
-        T * cv = a.carry + (uint64_t) (2 * ch) * a.R;
-        if(same) {
-          VT v = vzero<VT>();
-          if(r0 != CARRY_NONE) v += v0;
-          if(r1 != CARRY_NONE) v += v1;
-          v = group_allsum<T, V, L>(v);
-          if(g == 0) {
-            if(m != 0) vstore<T, V>(cv, 1u, a.R, col, cok, v);
-            // the chunk a carried row starts in clears it for the fix-up
-            if(m != 0 && a.covered && !cont) vstore<T, V>(a.out, ref, a.R, col, cok, vzero<VT>());
-            if(c == 0 && blockIdx.y == 0) {
-              a.carry_row[2 * ch] = CARRY_NONE;
-              a.carry_row[2 * ch + 1] = ref;
-            }
+        if(w1 != CARRY_NONE) {
+          vstore<T, V>(cv, 1u, a.R, col, cok, x1);
+          if(c == 0 && rowst) a.carry_row[2 * ch + 1] = w1;
+        }
+        // the chunk a carried row starts in clears it for the fix-up
+        if(a.covered) {
+          if(w0 != CARRY_NONE && !(cont && w0 == first_row)) {
+            vstore<T, V>(a.out, w0, a.R, col, cok, vzero<VT>());
           }
-        } else {
-          // through LDS: the records are dead once every group has walked
-          constexpr int NE = 2 * G;
-          static_assert(NE * CW * sizeof(T) <= NL * WS_WN * sizeof(uint32_t),
-              "the edge runs fit in the record space");
-          uint32_t * s_erow = s_orow[wave];
-          T * s_eval = reinterpret_cast<T *>(&s_tmp[wave][0][0]);
-          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-          __builtin_amdgcn_wave_barrier();
-          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-          s_erow[2 * g] = r0;
-          s_erow[2 * g + 1] = r1;
-          if(cok) {
-            *(VT *) (s_eval + (2 * g) * CW + c * V) = v0;
-            *(VT *) (s_eval + (2 * g + 1) * CW + c * V) = v1;
-          }
-          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-          __builtin_amdgcn_wave_barrier();
-          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-          if(g == 0) {
-            // the last group with positions holds the chunk's last run
-            uint32_t const glast = (wn + S - 1) / S - 1;
-            uint32_t rows[2];
-            combine_runs<T, V>(s_erow, s_eval, CW, 0, NE, true, 2 * glast + 1, rows, nullptr, 0,
-                a.out, a.R, col, c, cok, cv);
-            if(a.covered) {
-              #pragma unroll
-              for(int q=0; q < 2; ++q) {
-                if(rows[q] != CARRY_NONE && !(cont && rows[q] == first_row)) {
-                  vstore<T, V>(a.out, rows[q], a.R, col, cok, vzero<VT>());
-                }
-              }
-            }
-            if(c == 0 && blockIdx.y == 0) {
-              a.carry_row[2 * ch] = rows[0];
-              a.carry_row[2 * ch + 1] = rows[1];
-            }
+          if(w1 != CARRY_NONE && !(cont && w1 == first_row)) {
+            vstore<T, V>(a.out, w1, a.R, col, cok, vzero<VT>());
           }
         }
       }

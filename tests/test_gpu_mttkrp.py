@@ -398,3 +398,48 @@ def test_slice_edges_by_wave_size(gpu_available, small, prec):
                     assert rel(got, orc.mttkrp_coo(coo, m32, mode, f32=True)) <= TOL32, (R, mode)
     finally:
         L.spd_mttkrp_set_root_small(400000)
+
+
+@pytest.mark.parametrize("R", [4, 7, 8, 16, 40])
+@pytest.mark.parametrize("prec", [ps.F64, ps.F32])
+def test_short_slices_and_empty_rows(gpu_available, R, prec):
+    # slices of one to a few nonzeros, so that every wave ends many runs in
+    # every group, and outputs written without a fill: all rows in use, and
+    # tensors with unused rows at the end of a mode (cleared). The output
+    # starts as NaN.
+    print("case short slices", R, prec, flush=True)
+    L = ps.lib()
+    dt = np.float32 if prec == ps.F32 else np.float64
+    rng = np.random.default_rng(R)
+    n = 3001
+    i = np.sort(rng.integers(0, 1500, n))
+    i = np.unique(i, return_inverse=True)[1]
+    j = (np.arange(n) * 7) % 611
+    for extra in (0, 5):
+        inds = [i.astype(np.uint64), j.astype(np.uint64), (np.arange(n) % 1000).astype(np.uint64)]
+        vals = rng.lognormal(0.0, 1.0, n)
+        if extra:
+            inds[1] = inds[1] + 0
+            inds[1][-1] = 611 + extra          # rows 611 .. of mode 1 stay empty
+        dims = [int(x.max()) + 1 for x in inds]
+        coo = orc.Coo.from_arrays(inds, vals, dims)
+        mats = [ps.synth_matrix(d, R, 30 + m).astype(dt) for m, d in enumerate(dims)]
+        bufs = [ps.DevBuf.from_host(m) for m in mats]
+        arr = (ctypes.c_void_p * 3)(*[b.ptr for b in bufs])
+        for kind in (ps.CSF_ONEMODE, ps.CSF_ALLMODE):
+            opts = ps.Opts(csf_alloc=kind)
+            s = ps.CsfSet.convert(inds, vals, opts)
+            dims_in = [int(s.ptr[0].dims[m]) for m in range(3)]
+            assert dims_in == dims
+            for mode in range(3):
+                # an untiled root with empty rows writes slice positions
+                depth0 = int(s.ptr[mode if kind == ps.CSF_ALLMODE else 0].dim_perm[0])
+                if extra and depth0 == 1:
+                    continue
+                out = ps.DevBuf.from_host(np.full((dims[mode], R), np.nan, dtype=dt))
+                assert L.splatt_amd_mttkrp_dev(mode, R, s.ptr, arr, out.ptr, prec, opts.ptr,
+                                               None) == ps.SUCCESS
+                got = out.to_host((dims[mode], R), dt)
+                want = orc.mttkrp_coo(coo, mats, mode, f32=(prec == ps.F32))
+                assert np.all(np.isfinite(got)), (kind, mode)
+                assert rel(got, want) <= (TOL32 if prec == ps.F32 else TOL64), (kind, mode)
