@@ -363,15 +363,16 @@ wave_runs(uint32_t hrow, typename VecT<T, V>::type hval, uint32_t trow,
 // consecutive). One wave owns a chunk of FIX_CHUNK entries; group g of L
 // lanes loads entries g*FIX_CHUNK/G .. (g+1)*FIX_CHUNK/G - 1 at once and sums
 // their runs. A run closed on both sides inside a group is added to its row;
-// the groups' first and last runs are combined across the wave as in the
-// MTTKRP kernels (registers when they all belong to one row, LDS otherwise),
+// the groups' first and last runs are combined across the wave (wave_runs),
 // and the runs that reach the chunk's edges are added with one atomic
 // row-add each (a slice spanning P entries costs ~2P/FIX_CHUNK atomics on
 // its row). With a second-level buffer (carry2, crow2 not null) the chunk's
 // first and last runs go to its two entries there instead (the first run,
 // or none, then the last), and a second pass over those entries adds them:
 // a heavy row then sees ~4P/FIX_CHUNK^2 atomics instead of ~2P/FIX_CHUNK,
-// which long carry buffers need (atomics on one row serialise).
+// which long carry buffers need (atomics on one row serialise). Combining the
+// groups in registers instead of LDS: small tensor, three calls, 34.5 to 27.6
+// us; 50M-nonzero step 1383 to 1366.
 #define FIX_CHUNK 64
 // carry entries from which the fix-up takes two passes (4 modes, rank 64, 10M
 // nonzeros, 78000 entries a mode: 1080 to 1055 us a step)
@@ -392,11 +393,7 @@ k_root_fixup(T const * __restrict__ carry, uint32_t const * __restrict__ crow,
   typedef typename VecT<T, V>::type VT;
   constexpr int G = 64 / L;
   constexpr int EPG = FIX_CHUNK / G;           // entries per group
-  constexpr int CW = L * V;
   constexpr int NWB = MK_THREADS / 64;
-  __shared__ uint32_t s_erow[NWB][2 * G];
-  __shared__ __align__(16) T s_eval[NWB][2 * G][CW];
-  __shared__ __align__(16) T s_slot[NWB][2][CW];
   int const lane = threadIdx.x & 63;
   int const wave = threadIdx.x >> 6;
   uint32_t const c = lane % L;
@@ -443,7 +440,13 @@ k_root_fixup(T const * __restrict__ carry, uint32_t const * __restrict__ crow,
     acc += v[j];
   }
   VT const v1 = acc;
-  // the chunk's runs across the groups
+  // the chunk's runs across the groups. Runs closed inside the chunk are
+  // stored (they hold every partial of their row); the chunk's first run and
+  // the run of its last entry (it may continue past empty entries into the
+  // next chunk) leave it. An empty group lies between runs: the two entries
+  // of a wave or block that a run passes through are never both empty, and a
+  // group holds whole pairs.
+  static_assert(EPG % 2 == 0, "a pair of entries stays in one group");
   uint32_t const x = (r0 != CARRY_NONE) ? r0 : r1;
   uint64_t const m = __ballot(x != CARRY_NONE);
   if(m == 0) {                                // wave-uniform
@@ -453,60 +456,25 @@ k_root_fixup(T const * __restrict__ carry, uint32_t const * __restrict__ crow,
     }
     return;
   }
-  uint32_t const ref = __shfl(x, __ffsll((unsigned long long) m) - 1, 64);
-  bool const same = __all((r0 == CARRY_NONE || r0 == ref) && (r1 == CARRY_NONE || r1 == ref));
-  if(same) {
-    VT t = vzero<VT>();
-    if(r0 != CARRY_NONE) t += v0;
-    if(r1 != CARRY_NONE) t += v1;
-    t = group_allsum<T, V, L>(t);
-    if(two) {
-      // one run: it may continue on both sides
-      if(g == 0) vstore<T, V>(carry2, (uint32_t) (2 * wc + 1), R, col, cok, t);
-      if(rowst) {
-        crow2[2 * wc] = CARRY_NONE;
-        crow2[2 * wc + 1] = ref;
-      }
-    } else if(g == 0) {
-      vadd_atomic<T, V>(out, ref, R, col, skip, cok, t);
+  uint32_t const first_row = (uint32_t) __shfl((int) x, __ffsll((unsigned long long) m) - 1, 64);
+  uint32_t const lastg = (uint32_t) (63 - __clzll((long long) m)) / L;
+  uint32_t q0, q1;
+  VT x0, x1;
+  wave_runs<T, V, L>(r0, v0, r1, v1, first_row, true, lastg, out, R, col, cok, q0, x0, q1, x1);
+  bool const none0 = __ballot(q0 != CARRY_NONE) == 0;
+  if(two) {
+    if(rowst && none0) crow2[2 * wc] = CARRY_NONE;
+    if(q0 != CARRY_NONE) {
+      vstore<T, V>(carry2, (uint32_t) (2 * wc), R, col, cok, x0);
+      if(c == 0 && blockIdx.y == 0) crow2[2 * wc] = q0;
     }
-    return;
-  }
-  s_erow[wave][2 * g] = r0;
-  s_erow[wave][2 * g + 1] = r1;
-  if(cok) {
-    *(VT *) &s_eval[wave][2 * g][c * V] = v0;
-    *(VT *) &s_eval[wave][2 * g + 1][c * V] = v1;
-  }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  if(g == 0) {
-    // runs closed inside the chunk are stored (they hold every partial of
-    // their row); the chunk's first run and the run of its last entry (it
-    // may continue past empty entries into the next chunk) go to the slots
-    uint32_t el = 0;
-    for(int e=2 * G - 1; e >= 0; --e) {
-      if(s_erow[wave][e] != CARRY_NONE) {
-        el = (uint32_t) e;
-        break;
-      }
+    if(q1 != CARRY_NONE) {
+      vstore<T, V>(carry2, (uint32_t) (2 * wc + 1), R, col, cok, x1);
+      if(c == 0 && blockIdx.y == 0) crow2[2 * wc + 1] = q1;
     }
-    uint32_t rows[2];
-    combine_runs<T, V>(&s_erow[wave][0], &s_eval[wave][0][0], CW, 0, 2 * G, true, el,
-        rows, &s_slot[wave][0][0], CW, out, R, col, c, cok);
-    #pragma unroll
-    for(int q=0; q < 2; ++q) {
-      if(rows[q] != CARRY_NONE && cok) {
-        VT const sv = *(VT const *) &s_slot[wave][q][c * V];
-        if(two) vstore<T, V>(carry2, (uint32_t) (2 * wc + q), R, col, cok, sv);
-        else vadd_atomic<T, V>(out, rows[q], R, col, skip, cok, sv);
-      }
-    }
-    if(two && rowst) {
-      crow2[2 * wc] = rows[0];
-      crow2[2 * wc + 1] = rows[1];
-    }
+  } else {
+    if(q0 != CARRY_NONE) vadd_atomic<T, V>(out, q0, R, col, skip, cok, x0);
+    if(q1 != CARRY_NONE) vadd_atomic<T, V>(out, q1, R, col, skip, cok, x1);
   }
 }
 
@@ -1842,9 +1810,11 @@ extern "C" int spd_mttkrp_set_root_small(uint64_t nnz)
   return SPD_OK;
 }
 
-static uint32_t root3_wn(uint64_t nnz)
+// (Four times the carry rows: up to rank 512 they fit the scratch of the
+// allocation-free entry at any such size.)
+static uint32_t root3_wn(uint64_t nnz, uint64_t R)
 {
-  return (nnz <= g_r3_small && g_root_variant == 0) ? 64 : R3_WN;
+  return (nnz <= g_r3_small && R <= 512 && g_root_variant == 0) ? 64 : R3_WN;
 }
 
 // Lane layout (V columns per lane, L lanes per row chunk) for a rank R:
@@ -1898,7 +1868,7 @@ static int launch_root3(Root3Args<T> const & a, uint32_t nblocks, hipStream_t st
 {
   constexpr int CW = L * V;
   dim3 grid(nblocks, (unsigned) spd_cdiv(a.R, (uint64_t) CW));
-  bool const small = !HOIST && root3_wn(a.nnz) == 64;
+  bool const small = !HOIST && root3_wn(a.nnz, a.R) == 64;
   if constexpr (!HOIST) {
     if(small) {
       hipLaunchKernelGGL((k_root3<T, V, L, false, 1>), grid, dim3(R3_WAVES * 64), 0, st, a);
@@ -2277,7 +2247,7 @@ static int run_root3(spd_csf * c, uint64_t R, void * const * mats, void * out,
       c->nnz >= (uint64_t) R3_WN * 64) {
     return run_root3h<T>(c, R, mats, out, rows_pos, st, V, L, fx);
   }
-  uint32_t const WN = root3_wn(c->nnz);
+  uint32_t const WN = root3_wn(c->nnz, R);
   MttkrpPlan * plan = nullptr;
   if(fx == nullptr) {
     SPD_TRY(get_plan(c, WN, &plan, spd_hs(nullptr)));
