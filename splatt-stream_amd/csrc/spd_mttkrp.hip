@@ -1013,9 +1013,9 @@ vload_c(T const * __restrict__ base, uint32_t row, uint32_t R, uint32_t colc)
 // first and last runs returned in (r0, v0) and (r1, v1), as they may
 // continue in the neighbouring ranges; a range with one run returns it as
 // the last) or KIND_INTL/KIND_LEAF (every run added).
-template<typename T, int NG, int KIND, int V, int L, int B>
+template<typename T, int NG, int KIND, int V, int L, int B, int WN>
 __device__ __forceinline__ void
-walk_range(WsArgs<T> const & a, uint32_t const (*s_gid)[WS_WN], uint32_t const * s_orow,
+walk_range(WsArgs<T> const & a, uint32_t const (*s_gid)[WN], uint32_t const * s_orow,
     int32_t const * s_osl, T const * s_val, T * hot, uint32_t nhot, uint32_t k0, uint32_t k1,
     uint32_t c, uint32_t col, uint32_t colc, int skip, bool cok,
     uint32_t & r0, typename VecT<T, V>::type & v0, uint32_t & r1, typename VecT<T, V>::type & v1)
@@ -1164,7 +1164,8 @@ walk_range(WsArgs<T> const & a, uint32_t const (*s_gid)[WS_WN], uint32_t const *
 // FP32 root and copy walks of up to 4 modes run four waves per SIMD (batch
 // of 4, no spills); FP64, higher orders and the LDS-heavy internal and leaf
 // walks keep their registers.
-template<typename T, int N, int KIND, int V, int L, int B>
+// PER positions a lane: chunks of WN = 64 PER.
+template<typename T, int N, int KIND, int V, int L, int B, int PER>
 __global__ void __launch_bounds__(WS_WAVES * 64,
     (sizeof(T) == 4 && N <= 4 && (KIND == KIND_ROOT || KIND == KIND_COPY)) ? 4 : 1)
 k_walks(WsArgs<T> a)
@@ -1172,21 +1173,22 @@ k_walks(WsArgs<T> a)
   constexpr int NL = N - 1;                   // internal levels 0..N-2
   constexpr int NG = N - 1;                   // gathered levels per nonzero
   constexpr int G = 64 / L;
-  constexpr int S = WS_WN / G;
+  constexpr int WN = 64 * PER;
+  constexpr int LPW = 64 / PER;               // lanes per bitmap word
+  constexpr int S = WN / G;
   constexpr int CW = L * V;
-  constexpr int PER = WS_WN / 64;
   constexpr bool STRUCT = (KIND != KIND_COPY);          // stages the CSF structure
   constexpr bool PRIV = (KIND == KIND_INTL || KIND == KIND_LEAF);
   constexpr int WALK = (KIND == KIND_COPY) ? KIND_ROOT : KIND;
   constexpr int NLS = STRUCT ? NL : 1;
-  constexpr int HS = PRIV ? WS_WN : 1;
-  __shared__ uint32_t s_row[WS_WAVES][NLS][WS_WN];  // row id of local node k
+  constexpr int HS = PRIV ? WN : 1;
+  __shared__ uint32_t s_row[WS_WAVES][NLS][WN];  // row id of local node k
   // gathered row ids per position
-  __shared__ __align__(16) uint32_t s_tmp[WS_WAVES][NL][WS_WN];
-  __shared__ __align__(16) uint32_t s_orow[WS_WAVES][WS_WN];   // output row per position
+  __shared__ __align__(16) uint32_t s_tmp[WS_WAVES][NL][WN];
+  __shared__ __align__(16) uint32_t s_orow[WS_WAVES][WN];   // output row per position
   __shared__ int32_t s_osl[WS_WAVES][HS];           // its LDS slot
   __shared__ int32_t s_nsl[WS_WAVES][HS];           // slot of output-level node k
-  __shared__ __align__(16) T s_val[WS_WAVES][KIND == KIND_EXPAND ? 1 : WS_WN];
+  __shared__ __align__(16) T s_val[WS_WAVES][KIND == KIND_EXPAND ? 1 : WN];
   extern __shared__ __align__(16) unsigned char ws_dyn[];
   T * hot = (T *) ws_dyn;
 
@@ -1207,8 +1209,8 @@ k_walks(WsArgs<T> a)
   }
 
   for(uint32_t ch = blockIdx.x * WS_WAVES + wave; ch < a.nchunks; ch += gridDim.x * WS_WAVES) {
-    uint64_t const W0 = (uint64_t) ch * WS_WN;
-    uint64_t const W1 = (W0 + WS_WN < a.nnz) ? W0 + WS_WN : a.nnz;
+    uint64_t const W0 = (uint64_t) ch * WN;
+    uint64_t const W1 = (W0 + WN < a.nnz) ? W0 + WN : a.nnz;
     uint32_t const wn = (uint32_t) (W1 - W0);
     bool cont = false;             // the chunk's first row began in an earlier chunk
     if constexpr (!STRUCT) {
@@ -1216,9 +1218,9 @@ k_walks(WsArgs<T> a)
       // a row-sorted copy: records are stored as they are walked; each lane
       // copies PER consecutive positions with 16-byte loads and stores when
       // all of them lie in the chunk
-      static_assert(PER == 4, "the vector copy assumes 4 positions per lane");
+      static_assert(PER == 4 || PER == 1, "the copy takes one or four positions per lane");
       uint32_t const p0 = (uint32_t) lane * PER;
-      if(p0 + PER <= wn) {
+      if(PER == 4 && p0 + PER <= wn) {
         #pragma unroll
         for(int q=0; q < NG; ++q) {
           *(uint4 *) &s_tmp[wave][q][p0] = *(uint4 const *) (a.cg[q] + W0 + p0);
@@ -1247,29 +1249,32 @@ k_walks(WsArgs<T> a)
       uint32_t a0[NL], cnt[NL];
       uint32_t idx[NL][PER];
       {
-        uint32_t const wq = (uint32_t) lane >> 4;
-        uint32_t const sh = ((uint32_t) lane & 15u) * PER;
+        uint32_t const wq = (uint32_t) lane / LPW;
+        uint32_t const sh = ((uint32_t) lane % LPW) * PER;
         uint64_t const below = (1ull << sh) - 1ull;
-        uint64_t const wbase = ((uint64_t) ch * 4 + wq) * NL;
+        uint64_t const wbase = ((uint64_t) ch * PER + wq) * NL;
         #pragma unroll
         for(int l=0; l < NL; ++l) {
           a0[l] = a.plan[(uint64_t) ch * NL + l];
           uint2 const b2 = *(uint2 const *) (a.bits + wbase + l);
           uint64_t bw = (uint64_t) b2.x | ((uint64_t) b2.y << 32);
           if(l == 0) cont = (__builtin_amdgcn_readfirstlane((uint32_t) bw) & 1u) == 0u;
-          if(lane < 16) bw &= ~1ull;     // position 0 belongs to local node 0
+          if(lane < LPW) bw &= ~1ull;    // position 0 belongs to local node 0
           uint32_t const bc = (uint32_t) __popcll(bw);
-          uint32_t const c0 = __builtin_amdgcn_readlane(bc, 0), c1 = __builtin_amdgcn_readlane(bc, 16);
-          uint32_t const c2 = __builtin_amdgcn_readlane(bc, 32), c3 = __builtin_amdgcn_readlane(bc, 48);
-          uint32_t pre = (wq > 0 ? c0 : 0u) + (wq > 1 ? c1 : 0u) + (wq > 2 ? c2 : 0u) +
-                         (uint32_t) __popcll(bw & below);
-          uint32_t const b4 = (uint32_t) (bw >> sh) & 15u;
+          uint32_t pre = (uint32_t) __popcll(bw & below);
+          cnt[l] = 1u;
+          #pragma unroll
+          for(int w=0; w < PER; ++w) {
+            uint32_t const n = __builtin_amdgcn_readlane(bc, w * LPW);
+            pre += ((uint32_t) w < wq) ? n : 0u;
+            cnt[l] += n;
+          }
+          uint32_t const b4 = (uint32_t) (bw >> sh) & ((1u << PER) - 1u);
           #pragma unroll
           for(int q=0; q < PER; ++q) {
             pre += (b4 >> q) & 1u;
             idx[l][q] = pre;
           }
-          cnt[l] = 1u + c0 + c1 + c2 + c3;
         }
       }
       #pragma unroll
@@ -1293,7 +1298,10 @@ k_walks(WsArgs<T> a)
       T lv[PER];
       {
         uint32_t const p0 = (uint32_t) lane * PER;
-        if(p0 + PER <= wn) {
+        if constexpr (PER == 1) {
+          lf[0] = (p0 < wn) ? a.fids[N - 1][W0 + p0] : 0u;
+          if constexpr (KIND != KIND_EXPAND) lv[0] = (p0 < wn) ? a.vals[W0 + p0] : (T) 0;
+        } else if(p0 + PER <= wn) {
           uint4 const l4 = *(uint4 const *) (a.fids[N - 1] + W0 + p0);
           lf[0] = l4.x;
           lf[1] = l4.y;
@@ -1369,7 +1377,7 @@ k_walks(WsArgs<T> a)
       uint32_t r0, r1;
       VT v0 = vzero<VT>(), v1 = vzero<VT>();
       uint32_t const first_row = s_orow[wave][0];
-      walk_range<T, NG, WALK, V, L, B>(a, s_tmp[wave], s_orow[wave], s_osl[wave], s_val[wave],
+      walk_range<T, NG, WALK, V, L, B, WN>(a, s_tmp[wave], s_orow[wave], s_osl[wave], s_val[wave],
           hot, nhot, k0, k1, c, col, colc, skip, cok, r0, v0, r1, v1);
       if constexpr (WALK == KIND_ROOT) {
         // The chunk's edge runs: a run closed on both sides inside the chunk
@@ -1764,34 +1772,6 @@ static int get_plan(spd_csf * c, uint32_t S, MttkrpPlan ** out, hipStream_t st)
 
 // ---- dispatch -------------------------------------------------------------
 
-template<typename T, int N, int KIND, int V, int L>
-static int launch_walks(WsArgs<T> a, hipStream_t st)
-{
-  constexpr int CW = L * V;
-  constexpr int B = (N <= 4 && sizeof(T) == 8) ? 8 : 4;
-  uint32_t const ny = (uint32_t) spd_cdiv(a.R, (uint64_t) CW);
-  uint64_t nb = spd_cdiv(a.nchunks, WS_WAVES);
-  // Blocks that privatise rows in LDS are persistent (they fill and flush
-  // them once); root and copy walks take one chunk a wave: persistent, 1024
-  // blocks were 1.3 rounds of the three a CU that FP64 registers allow
-  // (ONEMODE rank 32, 10M nonzeros, three modes: 689 to 620 us).
-  if((KIND == KIND_INTL || KIND == KIND_LEAF) && nb > WS_BLOCKS) nb = WS_BLOCKS;
-  if(nb == 0) return SPD_OK;
-  size_t shmem = 0;
-  if constexpr (KIND == KIND_INTL || KIND == KIND_LEAF) {
-    uint32_t const cap = WS_HOT_BYTES / (CW * sizeof(T));
-    if(a.nhot > cap) a.nhot = cap;
-    shmem = (size_t) a.nhot * CW * sizeof(T);
-  }
-  hipLaunchKernelGGL((k_walks<T, N, KIND, V, L, B>), dim3((unsigned) nb, ny),
-      dim3(WS_WAVES * 64), shmem, st, a);
-  SPD_LAUNCH_CHECK();
-  if constexpr (KIND == KIND_ROOT || KIND == KIND_COPY) {
-    SPD_TRY((launch_fixup<T, V, L>(a.carry, a.carry_row, 2ull * a.nchunks, a.out, a.R, ny, st)));
-  }
-  return SPD_OK;
-}
-
 // 0: k_root3; 1: k_root3h with hot leaf rows in LDS; 2: k_root3h with
 // every row from HBM; 3: k_root3 gathering A once per fiber
 static int g_root_variant = 0;
@@ -1815,6 +1795,54 @@ extern "C" int spd_mttkrp_set_root_small(uint64_t nnz)
 static uint32_t root3_wn(uint64_t nnz, uint64_t R)
 {
   return (nnz <= g_r3_small && R <= 512 && g_root_variant == 0) ? 64 : R3_WN;
+}
+
+// The same for the root and copy walks of k_walks (two carry rows a chunk: up
+// to rank 128 they fit). All modes, 64 against 256: 9500 nonzeros in four modes
+// at FP32 rank 16 32.3 against 45.0 us, 113000 at rank 64 60.4 against 112.5,
+// 302000 at rank 35 89 against 122; between 7% slower and 39% faster over 44
+// tensors of up to 1.5M nonzeros, 8.6% on average.
+static uint32_t walks_wn(uint64_t nnz, uint64_t R)
+{
+  return (nnz <= g_r3_small && R <= 128) ? 64 : WS_WN;
+}
+
+template<typename T, int N, int KIND, int V, int L>
+static int launch_walks(WsArgs<T> a, hipStream_t st)
+{
+  constexpr int CW = L * V;
+  constexpr int B = (N <= 4 && sizeof(T) == 8) ? 8 : 4;
+  uint32_t const ny = (uint32_t) spd_cdiv(a.R, (uint64_t) CW);
+  uint64_t nb = spd_cdiv(a.nchunks, WS_WAVES);
+  // Blocks that privatise rows in LDS are persistent (they fill and flush
+  // them once); root and copy walks take one chunk a wave: persistent, 1024
+  // blocks were 1.3 rounds of the three a CU that FP64 registers allow
+  // (ONEMODE rank 32, 10M nonzeros, three modes: 689 to 620 us).
+  if((KIND == KIND_INTL || KIND == KIND_LEAF) && nb > WS_BLOCKS) nb = WS_BLOCKS;
+  if(nb == 0) return SPD_OK;
+  size_t shmem = 0;
+  if constexpr (KIND == KIND_INTL || KIND == KIND_LEAF) {
+    uint32_t const cap = WS_HOT_BYTES / (CW * sizeof(T));
+    if(a.nhot > cap) a.nhot = cap;
+    shmem = (size_t) a.nhot * CW * sizeof(T);
+  }
+  if constexpr (KIND == KIND_ROOT || KIND == KIND_COPY) {
+    if(walks_wn(a.nnz, a.R) == 64) {
+      hipLaunchKernelGGL((k_walks<T, N, KIND, V, L, B, 1>), dim3((unsigned) nb, ny),
+          dim3(WS_WAVES * 64), shmem, st, a);
+    } else {
+      hipLaunchKernelGGL((k_walks<T, N, KIND, V, L, B, 4>), dim3((unsigned) nb, ny),
+          dim3(WS_WAVES * 64), shmem, st, a);
+    }
+  } else {
+    hipLaunchKernelGGL((k_walks<T, N, KIND, V, L, B, 4>), dim3((unsigned) nb, ny),
+        dim3(WS_WAVES * 64), shmem, st, a);
+  }
+  SPD_LAUNCH_CHECK();
+  if constexpr (KIND == KIND_ROOT || KIND == KIND_COPY) {
+    SPD_TRY((launch_fixup<T, V, L>(a.carry, a.carry_row, 2ull * a.nchunks, a.out, a.R, ny, st)));
+  }
+  return SPD_OK;
 }
 
 // Lane layout (V columns per lane, L lanes per row chunk) for a rank R:
@@ -2343,7 +2371,7 @@ static int launch_expand(WsArgs<double> const & a, hipStream_t st)
   uint64_t nb = spd_cdiv(a.nchunks, WS_WAVES);
   if(nb > WS_BLOCKS) nb = WS_BLOCKS;
   if(nb == 0) return SPD_OK;
-  hipLaunchKernelGGL((k_walks<double, N, KIND_EXPAND, 1, 64, 1>), dim3((unsigned) nb),
+  hipLaunchKernelGGL((k_walks<double, N, KIND_EXPAND, 1, 64, 1, 4>), dim3((unsigned) nb),
       dim3(WS_WAVES * 64), 0, st, a);
   SPD_LAUNCH_CHECK();
   return SPD_OK;
@@ -2497,10 +2525,16 @@ static int run_mttkrp(spd_csf * c, int mode, uint64_t R, void * const * mats,
   }
   MttkrpPlan * plan = nullptr;
   // plans are built on the library stream; make the caller's stream wait
+  RowCopy * cp = nullptr;
+  if(depth > 0 && g_rowcopy) {
+    if(fx == nullptr) SPD_TRY(get_copy(c, depth, rows_pos, &cp, spd_hs(nullptr)));
+    else cp = find_copy(c, depth, rows_pos);
+  }
+  uint32_t const WN = (depth == 0 || cp != nullptr) ? walks_wn(c->nnz, R) : WS_WN;
   if(fx == nullptr) {
-    SPD_TRY(get_plan(c, WS_WN, &plan, spd_hs(nullptr)));
+    SPD_TRY(get_plan(c, WN, &plan, spd_hs(nullptr)));
     SPD_TRY(get_startbits(c, spd_hs(nullptr)));
-  } else if((plan = find_plan(c, WS_WN)) == nullptr || c->startbits == nullptr) {
+  } else if((plan = find_plan(c, WN)) == nullptr || c->startbits == nullptr) {
     return not_prepared("launch plan");
   }
   WsArgs<T> a = {};
@@ -2522,11 +2556,6 @@ static int run_mttkrp(spd_csf * c, int mode, uint64_t R, void * const * mats,
   a.R = (uint32_t) R;
   a.depth = depth;
   a.rows_are_positions = rows_pos;
-  RowCopy * cp = nullptr;
-  if(depth > 0 && g_rowcopy) {
-    if(fx == nullptr) SPD_TRY(get_copy(c, depth, rows_pos, &cp, spd_hs(nullptr)));
-    else cp = find_copy(c, depth, rows_pos);
-  }
   if(cp != nullptr) {
     for(int q=0; q < N - 1; ++q) a.cg[q] = cp->cg[q];
     a.crow = cp->crow;
@@ -2541,7 +2570,7 @@ static int run_mttkrp(spd_csf * c, int mode, uint64_t R, void * const * mats,
   // (everything above is built on the library stream and kept with the CSF)
   SpdCallScratch scratch(fx ? spd_hs(nullptr) : st);
   if(depth == 0 || cp != nullptr) {
-    // two partial rows per chunk of 256 positions, then the fix-up's second
+    // two partial rows per chunk, then the fix-up's second
     // level
     uint64_t const nent = 2ull * plan->nitems + fix_level2_entries(2ull * plan->nitems);
     void * cv = nullptr;

@@ -396,6 +396,21 @@ def test_slice_edges_by_wave_size(gpu_available, small, prec):
                     assert rel(got, orc.mttkrp_coo(coo, mats, mode)) <= TOL64, (R, mode)
                 else:
                     assert rel(got, orc.mttkrp_coo(coo, m32, mode, f32=True)) <= TOL32, (R, mode)
+        # the tree walks: roots and row-sorted copies of 4 and 5 modes
+        for dims, R in (([60, 40, 30, 20], 16), ([60, 40, 30, 20], 35), ([50, 20, 30, 9, 12], 8)):
+            inds, vals, dims = ps.synth_coord(dims, 7001, zipf=[1.1] + [0.0] * (len(dims) - 1),
+                                              vals="lognormal", seed=R)
+            coo = orc.Coo.from_arrays(inds, vals, dims)
+            mats = [ps.synth_matrix(d, R, 20 + m) for m, d in enumerate(dims)]
+            m32 = [m.astype(np.float32) for m in mats]
+            for kind in (ps.CSF_ONEMODE, ps.CSF_ALLMODE):
+                s = ps.CsfSet.convert(inds, vals, ps.Opts(csf_alloc=kind))
+                for mode in range(len(dims)):
+                    got = s.mttkrp(mode, mats)
+                    if prec == ps.F64:
+                        assert rel(got, orc.mttkrp_coo(coo, mats, mode)) <= TOL64, (dims, mode)
+                    else:
+                        assert rel(got, orc.mttkrp_coo(coo, m32, mode, f32=True)) <= TOL32, (dims, mode)
     finally:
         L.spd_mttkrp_set_root_small(400000)
 
