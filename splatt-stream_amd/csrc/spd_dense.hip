@@ -7,12 +7,12 @@
 //     16x16 output tiles of the upper triangle in registers and streams
 //     4-row slices of A through them; blocks write partial Grams that a
 //     second kernel sums in a fixed order (results are deterministic).
-//   - The R x R normal-equation matrix is formed, Cholesky-factored and
-//     inverted in one single-wave kernel (R^3/3 flops, latency-bound).
+//   - The R x R normal-equation matrix is formed and inverted in one
+//     workgroup, its entries in registers (R^3 flops, latency-bound).
 //   - The solve of every row against it (potrs in the reference) becomes a
-//     product with the inverse on MFMA, with the rows of the right-hand
-//     side staged through LDS; the column sums of squares needed for
-//     normalisation or the max-column-norm prox are fused into it.
+//     product with the inverse on MFMA, rows going from global memory to the
+//     matrix operands and back in registers; the column sums of squares
+//     needed for normalisation or the max-column-norm prox are fused into it.
 //   - Column reductions use fixed-order block partials, so repeated runs
 //     give bit-identical results.
 // Ranks up to 64 take the MFMA kernels; larger ranks take plain kernels.

@@ -3,8 +3,8 @@
 // (src/mttkrp.c:1287-1343 and the kernels at :390-1278).
 //
 // Work decomposition. The nonzeros (leaf level, in CSF order) are cut into
-// chunks of 256 consecutive nonzeros without regard to fiber or slice
-// boundaries, so a giant Zipf slice is spread over many chunks and every
+// chunks of 256 (64 in small tensors) consecutive nonzeros without regard to
+// fiber or slice boundaries, so a giant Zipf slice is spread over many chunks and every
 // chunk is the same amount of leaf work. A wavefront owns a chunk; it is
 // split between 64/L groups of L lanes, each lane holding V consecutive
 // columns of a factor row (a second grid dimension tiles wider ranks).
@@ -135,9 +135,9 @@ vadd_atomic(T * base, uint32_t row, uint32_t R, uint32_t col, int skip, bool ok,
 // test reads LDS. k_root3h (spd_root3h.hpp) is the persistent variant that
 // gathers A once per fiber and keeps the hottest B rows in LDS.
 // Slices completed inside an item are stored; the partial sums at item
-// edges are combined per wave and then per block (across lane groups in
-// registers when they all belong to one slice, through LDS otherwise), and
-// only a block's first and last slice (when they cross the block's edges)
+// edges are combined per wave (wave_runs) and then per block (across lane
+// groups in registers when they all belong to one slice, through LDS
+// otherwise), and only a block's first and last slice (when they cross the block's edges)
 // reach the carry buffer.
 
 #define R3_WAVES 4
