@@ -341,6 +341,9 @@ void spd_server_free(spd_server * sv);
  * (host/base.c; used by the server's per-stream sequences). */
 struct random_data;
 void spl_fill_rand_state(struct random_data * rd, double * vals, uint64_t n);
+/* Around every use of the process's generator (host/base.c). */
+void spl_rand_lock(void);
+void spl_rand_unlock(void);
 /* The values a server stream seeded with `seed` draws for its first n new
  * factor entries (for tests). */
 void spd_serve_rand_fill(unsigned seed, double * vals, uint64_t n);

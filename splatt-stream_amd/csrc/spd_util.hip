@@ -51,10 +51,13 @@ extern "C" int spd_init(void)
   // (the reference draws factors from rand(), src/util.c:15-40), and the
   // first device call may come after that seed, so the start-up runs on a
   // private generator state and the caller's state is put back untouched.
+  // Factor fills on other threads wait for it.
   static int32_t s_rand_state[32];
+  spl_rand_lock();
   char * const prev = initstate(1u, (char *) s_rand_state, sizeof(s_rand_state));
   int const rc = init_runtime();
   setstate(prev);
+  spl_rand_unlock();
   if(rc != SPD_OK) {
     return rc;
   }

@@ -91,13 +91,16 @@ splatt_error_type splatt_amd_set_mttkrp_layout(int layout)
 
 /* src/util.c:15-24: magnitude 3*rand()/RAND_MAX, negated when a second
  * rand() is even. Drawn on the host so the sequence is glibc's. */
+static val_t rand_value(int32_t a, int32_t b)
+{
+  val_t const v = 3.0 * ((val_t) a / (val_t) RAND_MAX);
+  return (b % 2 == 0) ? -v : v;
+}
+
 val_t spl_rand_val(void)
 {
-  val_t v = 3.0 * ((val_t) rand() / (val_t) RAND_MAX);
-  if(rand() % 2 == 0) {
-    v *= -1;
-  }
-  return v;
+  int32_t const a = rand();
+  return rand_value(a, rand());
 }
 
 /* n values from a glibc generator state, two draws each (as spl_rand_val).
@@ -111,8 +114,7 @@ void spl_fill_rand_state(struct random_data * rd, double * vals, uint64_t n)
       int32_t a = 0, b = 0;
       random_r(rd, &a);
       random_r(rd, &b);
-      double v = 3.0 * ((double) a / (double) RAND_MAX);
-      vals[i] = (b % 2 == 0) ? -v : v;
+      vals[i] = rand_value(a, b);
     }
     return;
   }
@@ -141,37 +143,163 @@ void spl_fill_rand_state(struct random_data * rd, double * vals, uint64_t n)
   rd->rptr = rptr;
 }
 
+/* One user of the process's generator at a time inside the library: the fills
+ * below, and the runtime's start-up, which runs beside it (spd_init). */
+static pthread_mutex_t rand_mu = PTHREAD_MUTEX_INITIALIZER;
+void spl_rand_lock(void)
+{
+  pthread_mutex_lock(&rand_mu);
+}
+void spl_rand_unlock(void)
+{
+  pthread_mutex_unlock(&rand_mu);
+}
+
+#define RAND_WORDS 32     /* the TYPE_3 state: a position and 31 words */
+#define RAND_BYTES (RAND_WORDS * sizeof(int32_t))
+#define RAND_PROBE 256    /* values a long fill draws with rand() first */
+#define RAND_LONG 2048    /* the shortest long fill */
+
+/* True if n successive rand() results of this thread are neighbours in one
+ * TYPE_3 sequence: o[i] = o[i-3] + o[i-31], but for a carry out of the lowest
+ * bits, which results do not show. A draw of another thread breaks it. */
+static int rand_undisturbed(uint32_t const * o, int n)
+{
+  for(int i=31; i < n; ++i) {
+    if(((o[i] - o[i - 3] - o[i - 31]) & 0x7fffffffu) > 1u) {
+      return 0;
+    }
+  }
+  return 1;
+}
+
+/* Moves the generator from its current state `live` to `cur`, which is not in
+ * use. A draw or a seed of another thread meanwhile changes `live`, which is
+ * then made current again and moved anew. */
+static void rand_move(int32_t * live, char * cur)
+{
+  int32_t sent[RAND_WORDS];
+  for(;;) {
+    memcpy(sent, live, RAND_BYTES);
+    memcpy(cur, sent, RAND_BYTES);
+    setstate(cur);
+    if(memcmp(live, sent, RAND_BYTES) == 0) {
+      return;
+    }
+    setstate((char *) live);
+  }
+}
+
+/* A copy of the process's state, which is out of use while its bytes are
+ * copied. 0 if another thread drew or seeded meanwhile (a seed is carried
+ * over) or the state is of another type. */
+static int rand_copy_state(int32_t * copy)
+{
+  static int32_t away[RAND_WORDS];     /* in use meanwhile */
+  int32_t same[RAND_WORDS];
+  struct random_data ra, rs, rc;
+  memset(&ra, 0, sizeof(ra));
+  memset(&rs, 0, sizeof(rs));
+  memset(&rc, 0, sizeof(rc));
+  initstate_r(1, (char *) away, RAND_BYTES, &ra);
+  initstate_r(1, (char *) same, RAND_BYTES, &rs);
+  initstate_r(1, (char *) copy, RAND_BYTES, &rc);
+  char * const cur = setstate((char *) away);
+  if(cur == NULL) {
+    return 0;
+  }
+  int ok = setstate_r(cur, &rc) == 0 && rc.rand_type == 3;
+  if(ok) {
+    memcpy(copy, cur, RAND_BYTES);
+  }
+  setstate(cur);
+  if(memcmp(away, same, RAND_BYTES) == 0) {
+    return ok;
+  }
+  /* draws alone lead on from where `away` began; after a seed they do not,
+   * and the seeded state is the process's */
+  for(int k=0; k < 4096; ++k) {
+    int32_t v;
+    random_r(&rs, &v);
+    if(memcmp(away + 1, same + 1, RAND_BYTES - sizeof(int32_t)) == 0) {
+      return 0;
+    }
+  }
+  if(ok) {
+    setstate((char *) away);
+    rand_move(away, cur);
+  }
+  return 0;
+}
+
+/* Makes `next` the process's state if that is still `seen`. */
+static int rand_commit_state(int32_t const * seen, int32_t * next)
+{
+  char * const cur = setstate((char *) next);
+  if(cur == NULL) {
+    return 0;
+  }
+  /* the position comes first; no state array is shorter than the two words */
+  if(memcmp(cur, seen, 2 * sizeof(int32_t)) != 0 || memcmp(cur, seen, RAND_BYTES) != 0) {
+    setstate(cur);
+    return 0;
+  }
+  rand_move(next, cur);
+  return 1;
+}
+
 /* Values of the process's rand() sequence, which goes on after them. rand()
- * itself takes a lock and a call per draw (a stream that adds 90000 rows of
- * rank 32 draws 6 million times: 113 ms against 10), so long fills run on the
- * generator's own state: a stand-in state is made current, which stores the
- * position of the caller's in its header, the draws are made from that, and
- * it is made current again. One fill at a time. */
+ * takes a lock and a call per draw (a stream that adds 90000 rows of rank 32
+ * draws 6 million times: 113 ms against 12), so a long fill draws from a copy
+ * of the generator's state and then moves the process's state on. The
+ * process's state stays in place meanwhile, and another thread may draw from
+ * it or seed it as beside a loop over rand(): if the first values show that
+ * one does, or the process's next draw is not the copy's first any more, the
+ * values are rand()'s. What is left are the two moments in which the state's
+ * bytes are copied (about 0.1 us each): a draw of another thread that falls
+ * into one may be out of sequence. */
 void spl_fill_rand(val_t * vals, idx_t nelems)
 {
-  static pthread_mutex_t mu = PTHREAD_MUTEX_INITIALIZER;
-  static char standin[128];
-  static char own[128];
+  static int32_t copy[RAND_WORDS];
   idx_t done = 0;
-  if(nelems >= 64) {
-    pthread_mutex_lock(&mu);
-    struct random_data rd;
-    memset(&rd, 0, sizeof(rd));
-    if(initstate_r(1, own, sizeof(own), &rd) == 0) {
-      char * const cur = initstate(1, standin, sizeof(standin));
-      if(cur != NULL) {
-        if(setstate_r(cur, &rd) == 0) {
-          spl_fill_rand_state(&rd, vals, nelems);
-          done = nelems;
-          /* stores the new position in cur's header */
-          setstate_r(own, &rd);
-        }
-        setstate(cur);
+  int ahead = 0;              /* a draw of the next value is already made */
+  int32_t first = 0;
+  spl_rand_lock();
+  if(nelems >= RAND_LONG) {
+    uint32_t o[2 * RAND_PROBE];
+    for(; done < RAND_PROBE; ++done) {
+      o[2 * done] = (uint32_t) rand();
+      o[2 * done + 1] = (uint32_t) rand();
+      vals[done] = rand_value((int32_t) o[2 * done], (int32_t) o[2 * done + 1]);
+    }
+    if(rand_undisturbed(o, 2 * RAND_PROBE) && rand_copy_state(copy)) {
+      struct random_data rd, rs;
+      int32_t own[RAND_WORDS], seen[RAND_WORDS];
+      int32_t expect = 0;
+      memset(&rd, 0, sizeof(rd));
+      memset(&rs, 0, sizeof(rs));
+      initstate_r(1, (char *) own, RAND_BYTES, &rd);
+      memcpy(seen, copy, RAND_BYTES);
+      setstate_r((char *) copy, &rd);
+      spl_fill_rand_state(&rd, vals + done, nelems - done);
+      setstate_r((char *) own, &rd);     /* stores the position in copy */
+      initstate_r(1, (char *) own, RAND_BYTES, &rs);
+      setstate_r((char *) seen, &rs);
+      random_r(&rs, &expect);
+      setstate_r((char *) own, &rs);
+      first = rand();
+      ahead = 1;
+      if(first == expect && rand_commit_state(seen, copy)) {
+        done = nelems;
+        ahead = 0;
       }
     }
-    pthread_mutex_unlock(&mu);
   }
-  for(idx_t i=done; i < nelems; ++i) {
-    vals[i] = spl_rand_val();
+  if(ahead) {
+    vals[done++] = rand_value(first, rand());
   }
+  for(; done < nelems; ++done) {
+    vals[done] = spl_rand_val();
+  }
+  spl_rand_unlock();
 }
