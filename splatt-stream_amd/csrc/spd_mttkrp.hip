@@ -180,8 +180,9 @@ struct Root3Args {
   T const * A;
   T const * B;
   T * out;
-  uint32_t const * plan;           // slice and fiber holding the first nonzero: per wave
-                                   // (k_root3), per item (k_root3h)
+  uint32_t const * plan;           // slice and fiber holding the first nonzero: a wave's at
+                                   // wid * pstride (k_root3), per item (k_root3h)
+  uint32_t pstride;
   uint8_t const * head;            // k_root3h: per item, its first slice began earlier
   uint64_t const * bits;           // per 64 nonzeros: slice-start word, fiber-start word
   T * carry;                       // 2 rows per block
@@ -575,7 +576,7 @@ k_root3(Root3Args<T> a)
   bool whead = false, wtail = false, ghead = false, gtail = false;
   bool longf = false;              // wave-uniform: few fibers in the wave
   if(wn > 0) {
-    uint2 const sf = *(uint2 const *) (a.plan + 2ull * wid);
+    uint2 const sf = *(uint2 const *) (a.plan + wid * a.pstride);
     S0 = sf.x;
     F0 = sf.y;
     // this lane's PER consecutive leaf ids and values, issued first: one
@@ -981,7 +982,8 @@ struct WsArgs {
   T const * vals;
   T const * gm[SPD_MAX_MODES];    // factor of the q-th gathered level, levels in order
   T * out;
-  uint32_t const * plan;          // per chunk: node at levels 0..N-2 holding its first nonzero
+  uint32_t const * plan;          // node at levels 0..N-2 holding a chunk's first nonzero:
+  uint32_t pstride;               // chunk ch's from ch * pstride
   uint64_t const * bits;          // node starts: per 64 nonzeros, one word per level < N-1
   int32_t const * hot_slot;       // internal/leaf: LDS slot of an output row (>= nhot: cold)
   uint32_t const * hot_rows;      // internal/leaf: output row of each LDS slot
@@ -1255,7 +1257,7 @@ k_walks(WsArgs<T> a)
         uint64_t const wbase = ((uint64_t) ch * PER + wq) * NL;
         #pragma unroll
         for(int l=0; l < NL; ++l) {
-          a0[l] = a.plan[(uint64_t) ch * NL + l];
+          a0[l] = a.plan[(uint64_t) ch * a.pstride + l];
           uint2 const b2 = *(uint2 const *) (a.bits + wbase + l);
           uint64_t bw = (uint64_t) b2.x | ((uint64_t) b2.y << 32);
           if(l == 0) cont = (__builtin_amdgcn_readfirstlane((uint32_t) bw) & 1u) == 0u;
@@ -1807,6 +1809,17 @@ static uint32_t walks_wn(uint64_t nnz, uint64_t R)
   return (nnz <= g_r3_small && R <= 128) ? 64 : WS_WN;
 }
 
+// Nonzeros an item of the launch plan takes: one plan serves waves of 64 and of
+// 256 (every fourth item), whatever the rank and the kernel.
+static uint32_t plan_items(uint64_t nnz)
+{
+  return nnz <= g_r3_small ? 64 : WS_WN;
+}
+static uint32_t plan_stride(spd_csf const * c, MttkrpPlan const * plan, uint32_t WN)
+{
+  return WN / plan->S * (uint32_t) (c->nmodes - 1);
+}
+
 template<typename T, int N, int KIND, int V, int L>
 static int launch_walks(WsArgs<T> a, hipStream_t st)
 {
@@ -2278,9 +2291,9 @@ static int run_root3(spd_csf * c, uint64_t R, void * const * mats, void * out,
   uint32_t const WN = root3_wn(c->nnz, R);
   MttkrpPlan * plan = nullptr;
   if(fx == nullptr) {
-    SPD_TRY(get_plan(c, WN, &plan, spd_hs(nullptr)));
+    SPD_TRY(get_plan(c, plan_items(c->nnz), &plan, spd_hs(nullptr)));
     SPD_TRY(get_startbits(c, spd_hs(nullptr)));
-  } else if((plan = find_plan(c, WN)) == nullptr || c->startbits == nullptr) {
+  } else if((plan = find_plan(c, plan_items(c->nnz))) == nullptr || c->startbits == nullptr) {
     return not_prepared("launch plan");
   }
   if(st != spd_hs(nullptr)) {
@@ -2311,6 +2324,7 @@ static int run_root3(spd_csf * c, uint64_t R, void * const * mats, void * out,
   a.B = (T const *) mats[c->perm[2]];
   a.out = (T *) out;
   a.plan = plan->nodes;
+  a.pstride = plan_stride(c, plan, WN);
   a.bits = c->startbits;
   a.carry = (T *) cv;
   a.carry_row = (uint32_t *) cr;
@@ -2403,7 +2417,7 @@ static int get_copy(spd_csf * c, int level, int rows_pos, RowCopy ** out, hipStr
   SPD_HIP(hipMemGetInfo(&fr, &tot));
   if(fr < 2 * (keep + temp) + (1ull << 30)) return SPD_OK;
   MttkrpPlan * plan = nullptr;
-  SPD_TRY(get_plan(c, WS_WN, &plan, st));
+  SPD_TRY(get_plan(c, plan_items(n), &plan, st));
   SPD_TRY(get_startbits(c, st));
   RowCopy * r = new RowCopy();
   r->level = level;
@@ -2433,9 +2447,10 @@ static int get_copy(spd_csf * c, int level, int rows_pos, RowCopy ** out, hipStr
     for(int q=0; q < NG; ++q) a.xg[q] = xg[q];
     a.xrow = xrow;
     a.plan = plan->nodes;
+    a.pstride = plan_stride(c, plan, WS_WN);
     a.bits = c->startbits;
     a.nnz = n;
-    a.nchunks = plan->nitems;
+    a.nchunks = (uint32_t) spd_cdiv(n, WS_WN);
     a.depth = level;
     a.rows_are_positions = rows_pos;
     switch(N) {
@@ -2532,9 +2547,9 @@ static int run_mttkrp(spd_csf * c, int mode, uint64_t R, void * const * mats,
   }
   uint32_t const WN = (depth == 0 || cp != nullptr) ? walks_wn(c->nnz, R) : WS_WN;
   if(fx == nullptr) {
-    SPD_TRY(get_plan(c, WN, &plan, spd_hs(nullptr)));
+    SPD_TRY(get_plan(c, plan_items(c->nnz), &plan, spd_hs(nullptr)));
     SPD_TRY(get_startbits(c, spd_hs(nullptr)));
-  } else if((plan = find_plan(c, WN)) == nullptr || c->startbits == nullptr) {
+  } else if((plan = find_plan(c, plan_items(c->nnz))) == nullptr || c->startbits == nullptr) {
     return not_prepared("launch plan");
   }
   WsArgs<T> a = {};
@@ -2550,9 +2565,10 @@ static int run_mttkrp(spd_csf * c, int mode, uint64_t R, void * const * mats,
   a.vals = (sizeof(T) == 4) ? (T const *) c->vals32 : (T const *) c->u.vals;
   a.out = (T *) out;
   a.plan = plan->nodes;
+  a.pstride = plan_stride(c, plan, WN);
   a.bits = c->startbits;
   a.nnz = c->nnz;
-  a.nchunks = plan->nitems;
+  a.nchunks = (uint32_t) spd_cdiv(c->nnz, WN);
   a.R = (uint32_t) R;
   a.depth = depth;
   a.rows_are_positions = rows_pos;
@@ -2570,9 +2586,8 @@ static int run_mttkrp(spd_csf * c, int mode, uint64_t R, void * const * mats,
   // (everything above is built on the library stream and kept with the CSF)
   SpdCallScratch scratch(fx ? spd_hs(nullptr) : st);
   if(depth == 0 || cp != nullptr) {
-    // two partial rows per chunk, then the fix-up's second
-    // level
-    uint64_t const nent = 2ull * plan->nitems + fix_level2_entries(2ull * plan->nitems);
+    // two partial rows per chunk, then the fix-up's second level
+    uint64_t const nent = 2ull * a.nchunks + fix_level2_entries(2ull * a.nchunks);
     void * cv = nullptr;
     void * cr = nullptr;
     if(fx != nullptr) {

@@ -14,6 +14,7 @@ import ctypes
 import numpy as np
 import pytest
 
+import oracle_py as orc
 import pysplatt as ps
 
 pytestmark = pytest.mark.gpu
@@ -86,4 +87,30 @@ def test_noalloc_rejects_unprepared_csf(gpu_available):
     finally:
         for b in dm:
             b.free()
+        s.free()
+
+
+@pytest.mark.parametrize("first,then", [(16, 200), (200, 16), (16, 600)])
+def test_noalloc_at_another_rank(gpu_available, first, then):
+    # root outputs need the launch plan and the start bitmaps alone, and both
+    # are the same for every rank: a CSF prepared at one rank serves others,
+    # on either side of the ranks up to which waves take 64 nonzeros
+    L = ps.lib()
+    for dims in ([60, 50, 40], [40, 30, 20, 12]):
+        print("case noalloc rank", first, then, len(dims), flush=True)
+        inds, vals, dims = ps.synth_coord(dims, 9000, zipf=[1.1] * len(dims), seed=15)
+        opts = ps.Opts(csf_alloc=ps.CSF_ALLMODE)
+        s = ps.CsfSet.convert(inds, vals, opts)
+        coo = orc.Coo.from_arrays(inds, vals, dims)
+        for R, fn in ((first, L.splatt_amd_mttkrp_dev), (then, L.splatt_amd_mttkrp_dev_noalloc)):
+            mats = [ps.synth_matrix(d, R, 70 + m) for m, d in enumerate(dims)]
+            dm = [ps.DevBuf.from_host(m) for m in mats]
+            try:
+                for mode in range(len(dims)):
+                    rc, got = _run(L, fn, s, opts, mode, R, dims, dm, ps.F64, np.float64)
+                    assert rc == ps.SUCCESS, ps.last_error()
+                    assert _rel(got, orc.mttkrp_coo(coo, mats, mode)) <= 1e-12
+            finally:
+                for b in dm:
+                    b.free()
         s.free()
