@@ -1437,13 +1437,16 @@ k_walks(WsArgs<T> a)
   }
 }
 
-// Row-sorted copy: position i of the copy is CSF position perm[i].
+// Row-sorted copy: position i of the copy is CSF position perm[i]. Hands the
+// sort's *holes on to the host (host_holes: pinned memory).
 __global__ void k_copy_gather(uint32_t const * __restrict__ perm, uint64_t n, int ng,
     DevPtrs32 xg, DevPtrs32 cg, double const * __restrict__ vals,
-    double * __restrict__ cv64, float * __restrict__ cv32)
+    double * __restrict__ cv64, float * __restrict__ cv32,
+    uint32_t const * __restrict__ holes, uint32_t * __restrict__ host_holes)
 {
   uint64_t i = (uint64_t) blockIdx.x * blockDim.x + threadIdx.x;
   uint64_t const stride = (uint64_t) gridDim.x * blockDim.x;
+  if(i == 0) *host_holes = *holes;
   for(; i < n; i += stride) {
     uint32_t const p = perm[i];
     for(int q=0; q < ng; ++q) cg.p[q][i] = xg.p[q][p];
@@ -1453,11 +1456,21 @@ __global__ void k_copy_gather(uint32_t const * __restrict__ perm, uint64_t n, in
   }
 }
 
-__global__ void k_u64_to_u32(uint64_t const * __restrict__ k, uint64_t n, uint32_t * __restrict__ o)
+// Sorted rows as 32-bit ids, and whether every row below nrows occurs: *holes
+// (zero before) is set by a row that does not follow its neighbour's.
+__global__ void k_sorted_rows(uint64_t const * __restrict__ k, uint64_t n, uint64_t nrows,
+    uint32_t * __restrict__ o, uint32_t * __restrict__ holes)
 {
   uint64_t i = (uint64_t) blockIdx.x * blockDim.x + threadIdx.x;
   uint64_t const stride = (uint64_t) gridDim.x * blockDim.x;
-  for(; i < n; i += stride) o[i] = (uint32_t) k[i];
+  bool hole = false;
+  for(; i < n; i += stride) {
+    uint64_t const r = k[i];
+    hole |= (i == 0) ? r != 0 : r > k[i - 1] + 1;
+    hole |= i + 1 == n && r + 1 != nrows;
+    o[i] = (uint32_t) r;
+  }
+  if(hole) *holes = 1u;
 }
 
 // ---- plans ----------------------------------------------------------------
@@ -2355,24 +2368,12 @@ extern "C" int spd_mttkrp_set_copies(int enable)
   return SPD_OK;
 }
 
-// Runs of equal values in a sorted array, one addition per wave.
-__global__ void __launch_bounds__(256)
-k_count_runs(uint32_t const * __restrict__ row, uint64_t n, uint32_t * __restrict__ out)
-{
-  uint64_t i = (uint64_t) blockIdx.x * blockDim.x + threadIdx.x;
-  uint64_t const stride = (uint64_t) gridDim.x * blockDim.x;
-  uint32_t cnt = 0;
-  for(; i < n; i += stride) cnt += (i == 0 || row[i] != row[i - 1]) ? 1u : 0u;
-  #pragma unroll
-  for(int o=32; o > 0; o >>= 1) cnt += __shfl_xor(cnt, o, 64);
-  if((threadIdx.x & 63) == 0 && cnt != 0) atomicAdd(out, cnt);
-}
-
 __global__ void k_sort_init(uint32_t const * __restrict__ row, uint64_t n,
-    uint64_t * __restrict__ key, uint32_t * __restrict__ val)
+    uint64_t * __restrict__ key, uint32_t * __restrict__ val, uint32_t * __restrict__ holes)
 {
   uint64_t i = (uint64_t) blockIdx.x * blockDim.x + threadIdx.x;
   uint64_t const stride = (uint64_t) gridDim.x * blockDim.x;
+  if(i == 0) *holes = 0u;
   for(; i < n; i += stride) {
     key[i] = row[i];
     val[i] = (uint32_t) i;
@@ -2416,6 +2417,15 @@ static int get_copy(spd_csf * c, int level, int rows_pos, RowCopy ** out, hipStr
   size_t fr = 0, tot = 0;
   SPD_HIP(hipMemGetInfo(&fr, &tot));
   if(fr < 2 * (keep + temp) + (1ull << 30)) return SPD_OK;
+  // one copy at a time writes the flag (its plain copy back to the host took
+  // some 25 us of a small tensor's first call)
+  static std::mutex flag_mu;
+  static uint32_t * host_holes = nullptr;
+  std::lock_guard<std::mutex> flag_lock(flag_mu);
+  if(host_holes == nullptr) {
+    SPD_HIP(hipHostMalloc((void **) &host_holes, sizeof(uint32_t), hipHostMallocPortable));
+  }
+  *host_holes = 1;
   MttkrpPlan * plan = nullptr;
   SPD_TRY(get_plan(c, plan_items(n), &plan, st));
   SPD_TRY(get_startbits(c, st));
@@ -2430,7 +2440,7 @@ static int get_copy(spd_csf * c, int level, int rows_pos, RowCopy ** out, hipStr
   for(int q=0; q < NG && rc == SPD_OK; ++q) rc = spd_malloc((void **) &xg[q], n * 4);
   for(int q=0; q < NG && rc == SPD_OK; ++q) rc = spd_malloc((void **) &r->cg[q], n * 4);
   if(rc == SPD_OK) rc = spd_malloc((void **) &xrow, n * 4);
-  if(rc == SPD_OK) rc = spd_malloc((void **) &r->crow, n * 4);
+  if(rc == SPD_OK) rc = spd_malloc((void **) &r->crow, (n + 1) * 4);
   if(rc == SPD_OK) rc = spd_malloc((void **) &r->v64, n * 8);
   if(rc == SPD_OK) rc = spd_malloc((void **) &r->v32, n * 4);
   if(rc == SPD_OK) rc = spd_malloc((void **) &k0, n * 8);
@@ -2463,10 +2473,12 @@ static int get_copy(spd_csf * c, int level, int rows_pos, RowCopy ** out, hipStr
     default: rc = SPD_EINPUT; break;
     }
   }
+  // behind the rows: whether some row does not occur
+  uint32_t * const d_holes = r->crow + n;
   int which = 0;
   if(rc == SPD_OK) {
     unsigned const grid = (unsigned) (spd_cdiv(n, 256) < 8192 ? spd_cdiv(n, 256) : 8192);
-    hipLaunchKernelGGL(k_sort_init, dim3(grid), dim3(256), 0, st, xrow, n, k0, v0);
+    hipLaunchKernelGGL(k_sort_init, dim3(grid), dim3(256), 0, st, xrow, n, k0, v0, d_holes);
     if(hipGetLastError() != hipSuccess) rc = SPD_EHIP;
     if(rc == SPD_OK) rc = spd_radix_sort(k0, v0, k1, v1, n, bits_of(c->dims[c->perm[level]]),
         &which, st);
@@ -2478,27 +2490,14 @@ static int get_copy(spd_csf * c, int level, int rows_pos, RowCopy ** out, hipStr
       src.p[q] = xg[q];
       dst.p[q] = r->cg[q];
     }
-    hipLaunchKernelGGL(k_u64_to_u32, dim3(grid), dim3(256), 0, st, which ? k1 : k0, n, r->crow);
+    hipLaunchKernelGGL(k_sorted_rows, dim3(grid), dim3(256), 0, st, which ? k1 : k0, n,
+        c->dims[c->perm[level]], r->crow, d_holes);
     hipLaunchKernelGGL(k_copy_gather, dim3(grid), dim3(256), 0, st, which ? v1 : v0, n, NG,
-        src, dst, c->u.vals, r->v64, r->v32);
+        src, dst, c->u.vals, r->v64, r->v32, d_holes, host_holes);
     if(hipGetLastError() != hipSuccess) rc = SPD_EHIP;
   }
-  // rows in use: run starts of the sorted rows (counted in a key buffer that
-  // the sort no longer needs)
-  uint32_t used = 0;
-  if(rc == SPD_OK) {
-    uint32_t * const d_used = (uint32_t *) (which ? k0 : k1);
-    unsigned const grid = (unsigned) (spd_cdiv(n, 256) < 1024 ? spd_cdiv(n, 256) : 1024);
-    rc = spd_zero_async(d_used, sizeof(uint32_t), st);
-    if(rc == SPD_OK) {
-      hipLaunchKernelGGL(k_count_runs, dim3(grid), dim3(256), 0, st, r->crow, n, d_used);
-      if(hipGetLastError() != hipSuccess) rc = SPD_EHIP;
-    }
-    if(rc == SPD_OK && hipMemcpyAsync(&used, d_used, sizeof(used), hipMemcpyDeviceToHost,
-          st) != hipSuccess) rc = SPD_EHIP;
-  }
   if(rc == SPD_OK) rc = (hipStreamSynchronize(st) == hipSuccess) ? SPD_OK : SPD_EHIP;
-  r->covered = (used == c->dims[c->perm[level]]);
+  r->covered = (*host_holes == 0);
   for(int q=0; q < NG; ++q) spd_free(xg[q]);
   spd_free(xrow);
   spd_free(k0); spd_free(k1); spd_free(v0); spd_free(v1);

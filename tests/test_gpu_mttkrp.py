@@ -458,3 +458,42 @@ def test_short_slices_and_empty_rows(gpu_available, R, prec):
                 want = orc.mttkrp_coo(coo, mats, mode, f32=(prec == ps.F32))
                 assert np.all(np.isfinite(got)), (kind, mode)
                 assert rel(got, want) <= (TOL32 if prec == ps.F32 else TOL64), (kind, mode)
+
+
+@pytest.mark.parametrize("hole", [None, 0, 150, 298])
+@pytest.mark.parametrize("wave", [64, 256])
+def test_copy_outputs_with_and_without_empty_rows(gpu_available, hole, wave):
+    # internal and leaf outputs over row-sorted copies: written without a fill
+    # when every row occurs; a first, middle or last but one row that does not
+    # occur is zero. The output starts as NaN.
+    print("case copy rows", hole, wave, flush=True)
+    L = ps.lib()
+    L.spd_mttkrp_set_root_small.argtypes = [ctypes.c_uint64]
+    rng = np.random.default_rng(5)
+    n, R = 4001, 12
+    dims = [20, 300, 500]
+    inds = [(np.arange(n) % 20), rng.permutation(np.arange(n) % 300), (np.arange(n) * 7) % 500]
+    if hole is not None:
+        for m in (1, 2):
+            inds[m] = np.where(inds[m] == hole, hole + 1, inds[m])
+    inds = [x.astype(np.uint64) for x in inds]
+    vals = rng.lognormal(0.0, 1.0, n)
+    coo = orc.Coo.from_arrays(inds, vals, dims)
+    mats = [ps.synth_matrix(d, R, 30 + m) for m, d in enumerate(dims)]
+    bufs = [ps.DevBuf.from_host(m) for m in mats]
+    arr = (ctypes.c_void_p * 3)(*[b.ptr for b in bufs])
+    opts = ps.Opts(csf_alloc=ps.CSF_ONEMODE)
+    assert L.spd_mttkrp_set_root_small(0 if wave == 256 else 1 << 40) == 0
+    try:
+        s = ps.CsfSet.convert(inds, vals, opts)
+        assert [int(s.ptr[0].dims[m]) for m in range(3)] == dims
+        for mode in range(3):
+            out = ps.DevBuf.from_host(np.full((dims[mode], R), np.nan))
+            assert L.splatt_amd_mttkrp_dev(mode, R, s.ptr, arr, out.ptr, ps.F64, opts.ptr,
+                                           None) == ps.SUCCESS
+            got = out.to_host((dims[mode], R), np.float64)
+            assert np.all(np.isfinite(got)), mode
+            assert rel(got, orc.mttkrp_coo(coo, mats, mode)) <= TOL64, mode
+        s.free()
+    finally:
+        L.spd_mttkrp_set_root_small(400000)
