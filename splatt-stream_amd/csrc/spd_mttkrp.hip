@@ -182,7 +182,6 @@ struct Root3Args {
   T * out;
   uint32_t const * plan;           // slice and fiber holding the first nonzero: a wave's at
                                    // wid * pstride (k_root3), per item (k_root3h)
-  uint32_t pstride;
   uint8_t const * head;            // k_root3h: per item, its first slice began earlier
   uint64_t const * bits;           // per 64 nonzeros: slice-start word, fiber-start word
   T * carry;                       // 2 rows per block
@@ -192,6 +191,7 @@ struct Root3Args {
   uint32_t nfibers;
   uint32_t nitems;
   uint32_t R;
+  uint32_t pstride;
   int rows_are_positions;
   int covered;                     // every output row has a slice: no fill ran before
 };
@@ -983,7 +983,7 @@ struct WsArgs {
   T const * gm[SPD_MAX_MODES];    // factor of the q-th gathered level, levels in order
   T * out;
   uint32_t const * plan;          // node at levels 0..N-2 holding a chunk's first nonzero:
-  uint32_t pstride;               // chunk ch's from ch * pstride
+                                  // chunk ch's from ch * pstride
   uint64_t const * bits;          // node starts: per 64 nonzeros, one word per level < N-1
   int32_t const * hot_slot;       // internal/leaf: LDS slot of an output row (>= nhot: cold)
   uint32_t const * hot_rows;      // internal/leaf: output row of each LDS slot
@@ -996,6 +996,7 @@ struct WsArgs {
   uint32_t nhot;
   uint64_t nnz;
   uint32_t nchunks;
+  uint32_t pstride;
   uint32_t R;
   int depth;                      // output level (internal, leaf and expand kernels)
   int rows_are_positions;         // level-0 row = node index
@@ -1163,9 +1164,9 @@ walk_range(WsArgs<T> const & a, uint32_t const (*s_gid)[WN], uint32_t const * s_
   }
 }
 
-// FP32 root and copy walks of up to 4 modes run four waves per SIMD (batch
-// of 4, no spills); FP64, higher orders and the LDS-heavy internal and leaf
-// walks keep their registers.
+// FP32 root and copy walks of up to 4 modes are held to four waves per SIMD
+// (batch of 4, no spills; three modes fit seven); FP64, higher orders and the
+// LDS-heavy internal and leaf walks keep their registers.
 // PER positions a lane: chunks of WN = 64 PER.
 template<typename T, int N, int KIND, int V, int L, int B, int PER>
 __global__ void __launch_bounds__(WS_WAVES * 64,
@@ -1257,7 +1258,7 @@ k_walks(WsArgs<T> a)
         uint64_t const wbase = ((uint64_t) ch * PER + wq) * NL;
         #pragma unroll
         for(int l=0; l < NL; ++l) {
-          a0[l] = a.plan[(uint64_t) ch * a.pstride + l];
+          a0[l] = a.plan[ch * a.pstride + l];
           uint2 const b2 = *(uint2 const *) (a.bits + wbase + l);
           uint64_t bw = (uint64_t) b2.x | ((uint64_t) b2.y << 32);
           if(l == 0) cont = (__builtin_amdgcn_readfirstlane((uint32_t) bw) & 1u) == 0u;
@@ -1378,7 +1379,6 @@ k_walks(WsArgs<T> a)
       uint32_t const k1 = (k0 + S < wn) ? k0 + S : wn;
       uint32_t r0, r1;
       VT v0 = vzero<VT>(), v1 = vzero<VT>();
-      uint32_t const first_row = s_orow[wave][0];
       walk_range<T, NG, WALK, V, L, B, WN>(a, s_tmp[wave], s_orow[wave], s_osl[wave], s_val[wave],
           hot, nhot, k0, k1, c, col, colc, skip, cok, r0, v0, r1, v1);
       if constexpr (WALK == KIND_ROOT) {
@@ -1389,6 +1389,7 @@ k_walks(WsArgs<T> a)
         // positions ends with a last run, so the chunk's last run is always
         // carried.
         T * const cv = a.carry + (uint64_t) (2 * ch) * a.R;
+        uint32_t const first_row = __builtin_amdgcn_readfirstlane(s_orow[wave][0]);
         uint32_t w0, w1;
         VT x0, x1;
         wave_runs<T, V, L>(r0, v0, r1, v1, first_row, true, (wn + S - 1) / S - 1, a.out, a.R, col,
@@ -1415,6 +1416,12 @@ k_walks(WsArgs<T> a)
         }
       }
     }
+    // one chunk a wave: without the loop the compiler does not lift the
+    // combine's lane offsets out of it and hold them over the walk (FP32, four
+    // modes: 128 VGPRs and spills to 104 and none, three modes 106 to 68; rank
+    // 64, 10M nonzeros, four modes 1072 to 1031 us a step). Chunks of 64 gain
+    // nothing (their few waves are latency-bound): 2% slower.
+    if constexpr (WALK == KIND_ROOT && PER == 4) break;
     // the next chunk's staging overwrites these records
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
