@@ -1733,7 +1733,7 @@ b_cpd_norm(GramSrc g, int nmodes, uint32_t R,
   if(t == 0) out[0] = fabs(s[0]);
 }
 
-__global__ void
+__global__ void __launch_bounds__(DN_THREADS)
 k_cpd_norm(GramSrc g, int nmodes, uint32_t R,
     double const * __restrict__ lambda, double * __restrict__ out)
 {
@@ -2822,7 +2822,7 @@ kb_admm_final(BSlot const * __restrict__ S, BHead const * __restrict__ hd, int m
 }
 
 // ||Z||^2 of the slice's model (time Gram of its one row) -> c->inner[1]
-__global__ void __launch_bounds__(64)
+__global__ void __launch_bounds__(DN_THREADS)
 kb_cpd_norm(BSlot const * __restrict__ S, BHead const * __restrict__ hd)
 {
   uint32_t const q = blockIdx.x;

@@ -13,7 +13,8 @@ READELF = "/opt/rocm/llvm/bin/llvm-readelf"
 
 
 def _kernels(tmp_path):
-    """Kernel name -> (VGPRs, scratch bytes) of every device code object."""
+    """Kernel name -> (VGPRs, scratch bytes, threads a block may have) of every
+    device code object."""
     with open(os.path.join(PKG, "libsplatt.so"), "rb") as f:
         data = f.read()
     found = {}
@@ -30,18 +31,31 @@ def _kernels(tmp_path):
                     return m.group(1) if m else None
                 if field("name") and field("vgpr_count"):
                     found[field("name")] = (int(field("vgpr_count")),
-                                            int(field("private_segment_fixed_size")))
+                                            int(field("private_segment_fixed_size")),
+                                            int(field("max_flat_workgroup_size")))
         at = data.find(b"\x7fELF", at + 4)
     return found
 
 
-@pytest.mark.skipif(not os.path.exists(READELF), reason="no llvm-readelf")
+pytestmark = pytest.mark.skipif(not os.path.exists(READELF), reason="no llvm-readelf")
+
+
+def test_norm_kernels_take_the_blocks_they_are_launched_with(tmp_path):
+    # the norm of the model is summed by 256 threads, alone and batched
+    seen = 0
+    for name, (_, _, threads) in _kernels(tmp_path).items():
+        if re.match(r"_Z\d+kb?_cpd_norm", name):
+            seen += 1
+            assert threads >= 256, name
+    assert seen == 2
+
+
 def test_fp32_walks_keep_their_registers(tmp_path):
     # root (0) and row-copy (4) walks of FP32 with 16-byte lanes over chunks
     # of 64 and 256 nonzeros: four waves per SIMD (512 / 4 VGPRs) without
     # scratch in four modes, five in three
     seen = 0
-    for name, (vgprs, scratch) in _kernels(tmp_path).items():
+    for name, (vgprs, scratch, _) in _kernels(tmp_path).items():
         m = re.match(r"_Z7k_walksIfLi([34])ELi[04]ELi4E", name)
         if m:
             seen += 1
