@@ -7,11 +7,12 @@
 // and the batch header (BHead). A kernel that the per-slice path launches
 // with nb(slice) blocks runs here as work items (slice s, block b < nb(s)):
 // each block of the batched launch computes nb(s) of every slice from the
-// slice's sizes, prefix-sums them in LDS, and strides over the items. Item
-// (s, b) executes exactly what block b of the per-slice launch executes
-// (same rows, same partial-sum slots, same reduction order), so a slice's
-// result does not depend on the other slices of its batch nor on the grid
-// of the batched launch.
+// slice's sizes, prefix-sums them in LDS, and strides over the items. What
+// item (s, b) computes (rows, partial-sum slots, reduction order) depends on
+// its slice alone, so a slice's result does not depend on the other slices
+// of its batch nor on the grid of the batched launch. Most items execute
+// what block b of the per-slice launch does; spd_dense.hip lists the steps
+// that differ.
 //
 // The outer ALS loop and the ADMM inner loop test their convergence on the
 // device: per slice flags in BCtl make later kernels skip a converged

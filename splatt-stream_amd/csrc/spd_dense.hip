@@ -601,6 +601,10 @@ k_gj_inv(GramSrc g, int nmodes, int mode, uint32_t R, double diag_add, int admm,
 }
 
 // ---- apply the inverse on MFMA (R <= 64) ---------------------------------------
+//
+// KIND 0: X = M G^{-1}; 1: the ADMM step before the proximal operator, with
+// column sums; 2: X += M G. Per slice only KIND 1 runs here (k_apply_reg has
+// the others); the batched launches run KIND 0 and 2.
 
 template<typename TM>
 struct ApplyArgs {
@@ -614,7 +618,8 @@ struct ApplyArgs {
   double * init;            // KIND 1
   double const * rho;       // KIND 1
   int clamp;                // KIND 1: column sums of max(P, 0)^2
-  double * colsq;           // per-block partial sums of squares (RP per block), or null
+  double * colsq;           // KIND 0 of k_apply_reg, KIND 1: per-block partial sums of
+                            // squares (RP per block), or null
 };
 
 template<int TT, typename TM, int KIND>
@@ -627,7 +632,7 @@ b_apply_mfma(ApplyArgs<TM> a,
   constexpr int RPI = (64 / RP) > 0 ? 64 / RP : 1;   // rows staged per pass
   __shared__ double s_g[RP * RP];
   __shared__ double s_m[4][16 * LD];
-  __shared__ double s_cs[RP];
+  __shared__ double s_cs[KIND == 1 ? RP : 1];
   int const lane = threadIdx.x & 63;
   int const wave = threadIdx.x >> 6;
   int const kk = lane >> 4;
@@ -635,7 +640,9 @@ b_apply_mfma(ApplyArgs<TM> a,
   uint64_t const I = a.I;
   uint32_t const R = a.R;
   for(int e=threadIdx.x; e < RP * RP; e += DN_THREADS) s_g[e] = a.ginv[e];
-  for(int e=threadIdx.x; e < RP; e += DN_THREADS) s_cs[e] = 0.;
+  if constexpr (KIND == 1) {
+    for(int e=threadIdx.x; e < RP; e += DN_THREADS) s_cs[e] = 0.;
+  }
   __syncthreads();
   double const rho = (KIND == 1) ? *a.rho : 0.;
   double cs[TT];
@@ -692,7 +699,6 @@ b_apply_mfma(ApplyArgs<TM> a,
           double const x = acc[t][r];
           if(KIND == 0) {
             a.X[idx] = x;
-            cs[t] += x * x;
           } else if(KIND == 2) {
             a.X[idx] += x;
           } else {
@@ -706,21 +712,23 @@ b_apply_mfma(ApplyArgs<TM> a,
       }
     }
   }
-  if(a.colsq != nullptr) {
-    #pragma unroll
-    for(int t=0; t < TT; ++t) {
-      cs[t] += __shfl_xor(cs[t], 16, 64);
-      cs[t] += __shfl_xor(cs[t], 32, 64);
-    }
-    for(int w=0; w < 4; ++w) {
-      if(wave == w && kk == 0) {
-        #pragma unroll
-        for(int t=0; t < TT; ++t) s_cs[t * 16 + cc] += cs[t];
+  if constexpr (KIND == 1) {
+    if(a.colsq != nullptr) {
+      #pragma unroll
+      for(int t=0; t < TT; ++t) {
+        cs[t] += __shfl_xor(cs[t], 16, 64);
+        cs[t] += __shfl_xor(cs[t], 32, 64);
       }
-      __syncthreads();
-    }
-    for(int e=threadIdx.x; e < RP; e += DN_THREADS) {
-      a.colsq[(uint64_t) blk * RP + e] = s_cs[e];
+      for(int w=0; w < 4; ++w) {
+        if(wave == w && kk == 0) {
+          #pragma unroll
+          for(int t=0; t < TT; ++t) s_cs[t * 16 + cc] += cs[t];
+        }
+        __syncthreads();
+      }
+      for(int e=threadIdx.x; e < RP; e += DN_THREADS) {
+        a.colsq[(uint64_t) blk * RP + e] = s_cs[e];
+      }
     }
   }
 }
@@ -2499,12 +2507,15 @@ extern "C" int spd_dense_admm_step(void const * M, int mdtype, double const * gi
 
 // ---- batched launches: one kernel covers every slice of a batch ----------
 //
-// Each kernel below runs the device body of its per-slice counterpart for
-// work item (slice s, block b), with b < nb(s) computed from the slice's
-// sizes by the same formula the per-slice launcher uses, so every slice
-// gets exactly its per-slice arithmetic (spd_batch.hpp). Items of slices
-// that a gate excludes (converged, other constraint kind, ...) are not
-// counted.
+// Each kernel below runs work item (slice s, block b) of a slice's dense
+// step, with b < nb(s) computed from the slice's sizes alone, so a slice's
+// result does not depend on its batch (spd_batch.hpp). The ADMM passes, the
+// inverse and the norm of the model run the per-slice bodies with the
+// per-slice block counts. Three steps do not, and differ from the per-slice
+// path in rounding: Grams (half as many blocks, bn_gram), row products
+// (b_apply_mfma here, k_apply_reg there) and column norms (kb_colreduce
+// here, k_colnorm_reduce there). Items of slices that a gate excludes
+// (converged, other constraint kind, ...) are not counted.
 
 #define BG_ALL 0          // every slice
 #define BG_LIVE 1         // slices whose outer loop runs
@@ -2519,7 +2530,7 @@ __host__ __device__ __forceinline__ uint32_t bn_clamp(uint64_t nb, uint64_t hi)
   if(nb > hi) nb = hi;
   return (uint32_t) nb;
 }
-// the block counts of the per-slice launchers
+// block counts: the per-slice launchers' but for bn_gram and bn_apply
 __host__ __device__ __forceinline__ uint32_t bn_gram(uint64_t I)
 {
   return bn_clamp(((I + 3) / 4 + 4 * GR_U * 4 - 1) / (4 * GR_U * 4), DN_MAX_BLOCKS);

@@ -118,13 +118,13 @@ vadd_atomic(T * base, uint32_t row, uint32_t R, uint32_t col, int skip, bool ok,
 // The hot path of an all-mode (or two-mode) CSF: out[s] = sum over fibers f
 // of slice s of A[fid(f)] o sum_{nnz j in f} v_j B[leaf(j)].
 //
-// A wave owns 256 consecutive nonzeros, split into G = 64/L items of 256/G
-// nonzeros (one per group of L lanes). Before walking, the wave stages into
+// A wave owns WN consecutive nonzeros (256; 64 of small tensors), split into
+// G = 64/L items of WN/G nonzeros (one per group of L lanes). Before walking, the wave stages into
 // LDS, with coalesced loads: the values and leaf ids of its nonzeros and the
 // id of every fiber and output row of every slice that overlaps its range.
 // Where fibers and slices start comes from two bitmaps built once per CSF
 // (one bit per nonzero: a fiber starts, a slice starts); a position's local
-// fiber and slice index is a population count over the wave's 256 bits. The
+// fiber and slice index is a population count over the wave's bits. The
 // bits at the groups' edges also tell which slices continue there, so nothing
 // is loaded after the walk, and the waves of a block keep their LDS apart
 // instead of sharing it behind a barrier (a wave holds its slot until it
@@ -147,7 +147,7 @@ vadd_atomic(T * base, uint32_t row, uint32_t R, uint32_t col, int skip, bool ok,
 // latencies (staging loads, then a gather a batch), so waves in flight count
 // more than loads a wave: 50M nonzeros, rank 32, FP32, all modes: 1497 us at
 // 6 gathers and 5 blocks, 1455 at 4 and 6 (with the long-fiber walk 1503 at 5
-// blocks, 1417 at 6).
+// blocks, 1417 at 6, where 16-byte lanes spill one register).
 #define R3_BATCH 4
 #define R3_OCC 6
 // Fibers times groups in a wave's 256 nonzeros up to which it skips the A
@@ -212,14 +212,13 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v)
 // Sum runs of equal rows over entries [e0, e1) (rows[e] == CARRY_NONE are
 // empty). The first run is "open" if open_first, the run containing entry
 // e_last is open at the end. Open runs go to slot 1 (open at the end) or
-// slot 0 (open at the start only) of (orow, oval) -- or, when oval is null,
-// to rows of carry (cv + slot*R, the caller's row range); closed runs are
-// stored to out. Empty slots report CARRY_NONE in orow.
+// slot 0 (open at the start only): its sum to row `slot` of cv, its row to
+// orow. Closed runs are stored to out. Empty slots report CARRY_NONE in orow.
 template<typename T, int V>
 __device__ __forceinline__ void
 combine_runs(uint32_t const * rows, T const * vals, int ld, uint32_t e0, uint32_t e1,
-    bool open_first, uint32_t e_last, uint32_t * orow, T * oval, int old_,
-    T * out, uint32_t R, uint32_t col, uint32_t c, bool cok, T * cv = nullptr)
+    bool open_first, uint32_t e_last, uint32_t * orow, T * out, uint32_t R, uint32_t col,
+    uint32_t c, bool cok, T * cv)
 {
   typedef typename VecT<T, V>::type VT;
   uint32_t cur = CARRY_NONE;
@@ -238,10 +237,7 @@ combine_runs(uint32_t const * rows, T const * vals, int ld, uint32_t e0, uint32_
           vstore<T, V>(out, cur, R, col, cok, acc);
         } else {
           if(slot == 0) r0 = cur; else r1 = cur;
-          if(cok) {
-            if(oval != nullptr) *(VT *) (oval + slot * old_ + c * V) = acc;
-            else vstore<T, V>(cv, (uint32_t) slot, R, col, cok, acc);
-          }
+          vstore<T, V>(cv, (uint32_t) slot, R, col, cok, acc);
         }
       }
       if(e == e1) break;
@@ -377,11 +373,13 @@ wave_runs(uint32_t hrow, typename VecT<T, V>::type hval, uint32_t trow,
 #define FIX_CHUNK 64
 // carry entries from which the fix-up takes two passes (4 modes, rank 64, 10M
 // nonzeros, 78000 entries a mode: 1080 to 1055 us a step)
-static uint64_t g_fix_two_level = 65536;
+#define FIX_TWO_LEVEL 65536
+static uint64_t g_fix_two_level = FIX_TWO_LEVEL;
 
+// (tests; UINT64_MAX: back to the default)
 extern "C" int spd_mttkrp_set_fix_two_level(uint64_t entries)
 {
-  g_fix_two_level = entries;
+  g_fix_two_level = (entries == UINT64_MAX) ? FIX_TWO_LEVEL : entries;
   return SPD_OK;
 }
 
@@ -566,7 +564,7 @@ k_root3(Root3Args<T> a)
 
   // ---- stage this wave's range ----
   // Each lane owns PER consecutive positions p = lane*PER + q, inside word
-  // lane/16 of the wave's four 64-position bitmap words. The local index of
+  // lane/LPW of the wave's PER bitmap words of 64 positions. The local index of
   // a position's fiber (slice) is the number of fiber (slice) starts at
   // positions 1..p; local index 0 is fiber F0 (slice S0), the one holding
   // the wave's first nonzero. Each position then gets its record.
@@ -716,8 +714,8 @@ k_root3(Root3Args<T> a)
   char const * const Bb = (char const *) a.B;
   char const * const Ab = (char const *) a.A;
   // the item's partial slices: H, the first slice when it began before the
-  // item and ends inside it or at its end (its sum goes to LDS entry e0 when
-  // it ends); T, the last slice when it continues past the item's end
+  // item and ends inside it or at its end; T, the last slice when it
+  // continues past the item's end
   uint32_t hrow = CARRY_NONE, trow = CARRY_NONE;
   VT tval = vzero<VT>();
   VT hval = vzero<VT>();
@@ -916,7 +914,7 @@ k_root3(Root3Args<T> a)
       }
     } else if(g == 0) {
       combine_runs<T, V>(&s_wrow[0][0], &s_wval[0][0][0], CW, 0, 2 * R3_WAVES,
-          block_head, 2 * lastw + 1, rows, nullptr, 0, a.out, R, col, c, cok, cv);
+          block_head, 2 * lastw + 1, rows, a.out, R, col, c, cok, cv);
     }
     // the fix-up adds to the carried rows: the block a carried slice starts
     // in clears its row
@@ -940,7 +938,8 @@ k_root3(Root3Args<T> a)
 // CSF order keeps the nonzeros of one output-level node contiguous, so a
 // group sums a run of equal output rows in registers and flushes it once.
 //
-// A wave owns chunks of 256 consecutive nonzeros (one, or with privatised rows
+// A wave owns chunks of WN consecutive nonzeros (256; 64 of small tensors in
+// root and copy walks; one chunk, or with privatised rows and in the expansion
 // those a persistent block strides over). Per chunk it stages into LDS, with coalesced loads, the
 // row ids and child pointers of every node of every level that overlaps the
 // chunk. Node starts are resolved bottom-up (a node starts where its first
@@ -1248,7 +1247,7 @@ k_walks(WsArgs<T> a)
       // holding W0 (from the plan), local node k >= 1 the k-th node starting
       // at a position 1..wn-1. A position's local node index is the number
       // of starts at positions 1..p, counted in the level's bitmap words
-      // (lane owns positions 4*lane..4*lane+3, inside word lane/16).
+      // (lane owns positions PER * lane .., inside word lane / LPW).
       uint32_t a0[NL], cnt[NL];
       uint32_t idx[NL][PER];
       {
@@ -1806,9 +1805,10 @@ static int g_root_variant = 0;
 // 37.6 (uniform: even at 300k to 500k).
 #define R3_SMALL_NNZ 400000
 static uint64_t g_r3_small = R3_SMALL_NNZ;
+// (tests; UINT64_MAX: back to the default)
 extern "C" int spd_mttkrp_set_root_small(uint64_t nnz)
 {
-  g_r3_small = nnz;
+  g_r3_small = (nnz == UINT64_MAX) ? R3_SMALL_NNZ : nnz;
   return SPD_OK;
 }
 
