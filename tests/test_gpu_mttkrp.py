@@ -24,6 +24,7 @@ pytestmark = pytest.mark.gpu
 
 TOL64 = 1e-12
 TOL32 = 1e-5
+DEFAULT = (1 << 64) - 1          # the dispatch limits' setters: back to the default
 
 
 def rel(a, b):
@@ -200,7 +201,7 @@ def test_slice_edges(gpu_available, prec, layout):
 
 def test_slice_edges_two_level_fixup(gpu_available):
     # the carry fix-up's two-pass form (taken by long carry buffers, from
-    # 131072 entries) forced on every size
+    # 65536 entries) forced on every size
     L = ps.lib()
     L.spd_mttkrp_set_fix_two_level.argtypes = [ctypes.c_uint64]
     assert L.spd_mttkrp_set_fix_two_level(0) == 0
@@ -210,7 +211,7 @@ def test_slice_edges_two_level_fixup(gpu_available):
         _set_precision(ps.F64)
         test_heavy_zipf_slices(gpu_available, ps.LAYOUT_AUTO)
     finally:
-        L.spd_mttkrp_set_fix_two_level(131072)
+        L.spd_mttkrp_set_fix_two_level(DEFAULT)
         _set_precision(ps.F64)
         _set_layout(ps.LAYOUT_AUTO)
 
@@ -412,7 +413,7 @@ def test_slice_edges_by_wave_size(gpu_available, small, prec):
                     else:
                         assert rel(got, orc.mttkrp_coo(coo, m32, mode, f32=True)) <= TOL32, (dims, mode)
     finally:
-        L.spd_mttkrp_set_root_small(400000)
+        L.spd_mttkrp_set_root_small(DEFAULT)
 
 
 @pytest.mark.parametrize("R", [4, 7, 8, 16, 40])
@@ -496,4 +497,61 @@ def test_copy_outputs_with_and_without_empty_rows(gpu_available, hole, wave):
             assert rel(got, orc.mttkrp_coo(coo, mats, mode)) <= TOL64, mode
         s.free()
     finally:
-        L.spd_mttkrp_set_root_small(400000)
+        L.spd_mttkrp_set_root_small(DEFAULT)
+
+
+@pytest.mark.parametrize("two_level", [False, True])
+@pytest.mark.parametrize("wave", [64, 256])
+@pytest.mark.parametrize("prec", [ps.F64, ps.F32])
+def test_every_output_row_is_written(gpu_available, prec, wave, two_level):
+    # outputs start as NaN: root and copy outputs with and without a fill
+    # before them, at both wave sizes and both forms of the fix-up. One row of
+    # every mode holds a third of the nonzeros (it spans many blocks and is
+    # carried), the others a few; untiled with every row in use, and tiled
+    # with row ids and rows that do not occur, the root's among them.
+    print("case written", prec, wave, two_level, flush=True)
+    L = ps.lib()
+    L.spd_mttkrp_set_root_small.argtypes = [ctypes.c_uint64]
+    L.spd_mttkrp_set_fix_two_level.argtypes = [ctypes.c_uint64]
+    dt = np.float32 if prec == ps.F32 else np.float64
+    rng = np.random.default_rng(21)
+    n, R = 9001, 9
+    assert L.spd_mttkrp_set_root_small(0 if wave == 256 else 1 << 40) == 0
+    assert L.spd_mttkrp_set_fix_two_level(0 if two_level else DEFAULT) == 0
+    try:
+        for full in ([701, 499, 302], [401, 299, 102, 53]):
+            for tiled in (False, True):
+                inds = []
+                for m, d in enumerate(full):
+                    x = rng.permutation(np.arange(n) % d)
+                    x[rng.permutation(n)[:n // 3]] = 7 + m
+                    x[:d] = np.arange(d)
+                    if tiled:
+                        x[x % 10 == 3] = d - 1
+                    inds.append(x.astype(np.uint64))
+                vals = rng.lognormal(0.0, 1.0, n)
+                coo = orc.Coo.from_arrays(inds, vals, full)
+                mats = [ps.synth_matrix(d, R, 80 + m).astype(dt) for m, d in enumerate(full)]
+                bufs = [ps.DevBuf.from_host(m) for m in mats]
+                arr = (ctypes.c_void_p * len(full))(*[b.ptr for b in bufs])
+                for kind in (ps.CSF_ONEMODE, ps.CSF_ALLMODE):
+                    opts = ps.Opts(csf_alloc=kind, tile=ps.DENSETILE, tilelevel=1, nthreads=5) \
+                        if tiled else ps.Opts(csf_alloc=kind)
+                    s = ps.CsfSet.convert(inds, vals, opts)
+                    assert [int(s.ptr[0].dims[m]) for m in range(len(full))] == full
+                    for mode, d in enumerate(full):
+                        out = ps.DevBuf.from_host(np.full((d + 1, R), np.nan, dtype=dt))
+                        assert L.splatt_amd_mttkrp_dev(mode, R, s.ptr, arr, out.ptr, prec,
+                                                       opts.ptr, None) == ps.SUCCESS
+                        got = out.to_host((d + 1, R), dt)
+                        want = orc.mttkrp_coo(coo, mats, mode, f32=(prec == ps.F32))
+                        what = (full, tiled, kind, mode)
+                        assert np.all(np.isnan(got[d])), what
+                        assert np.all(np.isfinite(got[:d])), what
+                        assert rel(got[:d], want) <= (TOL32 if prec == ps.F32 else TOL64), what
+                    s.free()
+                for b in bufs:
+                    b.free()
+    finally:
+        L.spd_mttkrp_set_root_small(DEFAULT)
+        L.spd_mttkrp_set_fix_two_level(DEFAULT)
