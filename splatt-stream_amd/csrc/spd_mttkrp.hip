@@ -574,7 +574,7 @@ k_root3(Root3Args<T> a)
   bool whead = false, wtail = false, ghead = false, gtail = false;
   bool longf = false;              // wave-uniform: few fibers in the wave
   if(wn > 0) {
-    uint2 const sf = *(uint2 const *) (a.plan + wid * a.pstride);
+    uint2 const sf = *(uint2 const *) (a.plan + (uint32_t) wid * a.pstride);
     S0 = sf.x;
     F0 = sf.y;
     // this lane's PER consecutive leaf ids and values, issued first: one
